@@ -386,6 +386,7 @@ int fecx_create(fecx_ctx** out, int device) {
     (void)dev(ctx, "flag", sizeof(int));
     if (device >= 0) {
       HIPCHK(hipHostMalloc((void**)&ctx->flag_host, sizeof(int), hipHostMallocDefault));
+      HIPCHK(hipHostMalloc((void**)&ctx->cg_done_host, sizeof(int), hipHostMallocDefault));
       // the allocation-free entry point's per-device scratch address, looked up once per device, device current
       require(fecx::noalloc_setup(device) == FECX_OK, FECX_ERR_HIP, "scratch symbol lookup failed");
     }
@@ -401,8 +402,10 @@ int fecx_destroy(fecx_ctx* ctx) {
   for (auto& kv : ctx->buf)
     if (kv.second.p) (void)hipFree(kv.second.p);
   for (hipEvent_t e : ctx->events) (void)hipEventDestroy(e);
+  for (hipEvent_t e : ctx->cg_events) (void)hipEventDestroy(e);
   if (ctx->stream2) (void)hipStreamDestroy(ctx->stream2);
   if (ctx->flag_host) (void)hipHostFree(ctx->flag_host);
+  if (ctx->cg_done_host) (void)hipHostFree(ctx->cg_done_host);
   delete ctx;
   return FECX_OK;
 }

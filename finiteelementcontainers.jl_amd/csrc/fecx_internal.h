@@ -273,6 +273,9 @@ struct fecx_ctx {
   // cleared on the device only when the last read-back did not find it clear (an error, or a call that stopped early)
   int* flag_host = nullptr;
   bool flag_dirty = true;
+  // conjugate gradients: pinned convergence word and the events that mark the enqueued batches of iterations
+  int* cg_done_host = nullptr;
+  std::vector<hipEvent_t> cg_events;
   // profiling
   bool profiling = false;
   std::vector<std::string> prof_names;

@@ -1,0 +1,89 @@
+"""The SpMV and the two-kernel CG iteration over every row form they dispatch on (1, 2 or 3 fields per node, the dof-level CSR
+of a Dirichlet set that splits nodes), at the sizes where lane groups and work-group ranges end: a single unknown node, rows
+narrower and far wider than a lane group's pass, unknown counts around the work-group sizes.
+
+Tolerances, derived beforehand: SpMV sums at most ~500 products, |error| <= 500 eps (|A| |x|) row by row with
+eps = 2^-53; a CG of 8 iterations on a mass matrix (condition number below ~1e2 after Jacobi scaling) amplifies the
+FP64 rounding of its dot products by at most its condition number per iteration, well under 1e-9 of the iterate."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _mesh(fec, name):
+    """(mesh, nf, fixed nodes per component)"""
+    if name.startswith("quad4"):
+        n = int(name.split()[1])
+        m = fec.StructuredMesh("quad", (0.0, 0.0), (1.0, 1.0), (n + 1, n + 1))
+        return m, 2 if "nf2" in name else 1, {}
+    if name == "hex8 one node":  # 2^3 elements, every node fixed but the centre
+        m = fec.StructuredMesh("hex", (0.0,) * 3, (1.0,) * 3, (3, 3, 3))
+        edge = fec.boundary_nodes(m)
+        return m, 3, {0: edge, 1: edge, 2: edge}
+    if name.startswith("hex8"):
+        n = int(name.split()[1])
+        m = fec.StructuredMesh("hex", (0.0,) * 3, (1.0,) * 3, (n + 1,) * 3)
+        fixed = {d: np.flatnonzero(m.coords[:, d] < 1e-12) + 1 for d in range(3)} if "roller" in name else {}
+        return m, 1 if "nf1" in name else 3, fixed
+    return fec.fan_tet10_mesh(int(name.split()[1])), 1 if "nf1" in name else 3, {}
+
+
+CASES = ["quad4 1", "quad4 7", "quad4 31 nf2", "hex8 one node", "hex8 1", "hex8 6", "hex8 9 nf1", "hex8 14", "hex8 5 roller",
+         "fan 5", "fan 32", "fan 32 nf1"]
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_spmv_and_cg_iterations(fec, gpu, name):
+    print(f"[krylov] {name}", flush=True)
+    mesh, nf, fixed = _mesh(fec, name)
+    space = fec.FunctionSpace(mesh, "H1Field", "Lagrange")
+    var = fec.ScalarFunction(space, "u") if nf == 1 else fec.VectorFunction(space, "displ")
+    asm = fec.SparseMatrixAssembler(var, sparse_matrix_type="csr", device=0)
+    for d, nodes in fixed.items():
+        mesh.nodeset_nodes[f"_f{d}"] = nodes
+    bcs = [fec.DirichletBC(var.names[d], lambda X, t: 0.0, nset_name=f"_f{d}") for d in fixed]
+    physics = fec.Poisson() if nf == 1 else fec.Mechanics(fec.PlaneStrain() if nf == 2 else None)
+    p = fec.create_parameters(mesh, asm, physics, dirichlet_bcs=bcs)
+    Uu = fec.create_unknowns(asm)
+    fec.assemble_mass_(asm, fec.mass, Uu, p)
+    M = fec.mass(asm)
+    A = M.to_scipy()
+    n = A.shape[0]
+    g = np.random.default_rng(1)
+    # SpMV with arbitrary values on the pattern
+    vals = torch.from_numpy(g.standard_normal(asm.nnz)).to(gpu)
+    x = g.standard_normal(n)
+    y = torch.full_like(Uu, np.nan)
+    xd = torch.from_numpy(x).to(gpu)
+    asm.ctx.call("fecx_csr_spmv", fec.assembler._ptr(vals), fec.assembler._ptr(xd), fec.assembler._ptr(y))
+    B = A.copy()
+    B.data = vals.cpu().numpy()
+    bound = 500 * 2.0 ** -53 * (abs(B) @ np.abs(x)) + 1e-300
+    assert np.all(np.abs(y.cpu().numpy() - B @ x) <= bound)
+    # eight CG iterations on the mass matrix from a nonzero start, with and without the preconditioner
+    b = g.standard_normal(n)
+    bd = torch.from_numpy(b).to(gpu)
+    for pre in (1, 0):
+        xg = torch.from_numpy(x).to(gpu)
+        it, res = ctypes.c_int(-1), ctypes.c_double(-1.0)
+        asm.ctx.call("fecx_cg_solve", fec.assembler._ptr(M.values), fec.assembler._ptr(bd), fec.assembler._ptr(xg),
+                     ctypes.c_double(1e-9), ctypes.c_double(0.0), ctypes.c_int(8), ctypes.c_int(pre), ctypes.byref(it),
+                     ctypes.byref(res))
+        d = 1.0 / A.diagonal() if pre else np.ones(n)
+        xs, r = x.copy(), b - A @ x
+        z = d * r
+        q, rz, k = z.copy(), r @ z, 0
+        while k < 8 and np.linalg.norm(r) > 1e-9 * np.linalg.norm(b):
+            Aq = A @ q
+            a = rz / (q @ Aq)
+            xs, r = xs + a * q, r - a * Aq
+            z = d * r
+            new = r @ z
+            q, rz, k = z + new / rz * q, new, k + 1
+        assert it.value == k
+        assert np.linalg.norm(xg.cpu().numpy() - xs) <= 1e-9 * np.linalg.norm(xs)
+        assert abs(res.value - np.linalg.norm(r)) <= 1e-9 * np.linalg.norm(b)
