@@ -359,7 +359,11 @@ void assemble_mass(fecx_ctx* ctx, int what, double density, const double* V, dou
   fecx::ReduceArgs ra = reduce_args(ctx);
   ra.R = R;
   ra.vals = (ctx->partial && vals) ? get<double>(ctx, "vals_full") : vals;
-  prof.run("reduce", ctx->stream, [&] { rc = fecx::launch_reduce(ctx->nf, ra, ctx->stream); });
+  const bool expand = what == fecx::MASS_MATRIX && ctx->nf > 1;  // one word per node pair: the blocks are m I
+  if (expand) ra.kel_off = get<int16_t>(ctx, "kel_off1");
+  prof.run("reduce", ctx->stream, [&] {
+    rc = expand ? fecx::launch_reduce_expand(ctx->nf, ra, ctx->stream) : fecx::launch_reduce(ctx->nf, ra, ctx->stream);
+  });
   require(rc == 0, FECX_ERR_UNSUPPORTED, "no reduction kernel for this element kind / nf");
   HIPCHK(hipGetLastError());
   compact_values(ctx, ra.vals, vals);
@@ -645,6 +649,11 @@ int fecx_build_pattern(fecx_ctx* ctx, int64_t* nnz) {
               (int16_t)(fecx::pair_pos(nnpe, la, b, pr.slot) * nf * nf + (pr.ab ? c : (c % nf) * nf + c / nf));
         }
       upload(ctx, "kel_off", off);
+      std::vector<int16_t> off1((size_t)nnpe * nnpe);  // the same for one word per pair (mass matrices of any nf)
+      for (int la = 0; la < nnpe; ++la)
+        for (int b = 0; b < nnpe; ++b)
+          off1[(size_t)la * nnpe + b] = (int16_t)fecx::pair_pos(nnpe, la, b, fecx::pair_ref(nnpe, la, b).slot);
+      upload(ctx, "kel_off1", off1);
     }
     dev(ctx, "Rel", sizeof(float) * ctx->ne * ctx->nnpe * nf);
     dev(ctx, "Kel", sizeof(float) * ctx->ne * ctx->pairs.npairs * nf * nf);

@@ -121,7 +121,7 @@ struct MatParams {
 
 enum Mode { MODE_R = 1, MODE_K = 2, MODE_ACTION_MF = 4, MODE_ACTION_ASM = 8, MODE_QPGRAD = 16, MODE_DIAG = 32 };
 
-// mass-type assemblies (mass.hip): consistent mass blocks into Kel; lumped mass, mass diagonal or mass action into Rel
+// mass-type assemblies (mass.hip): consistent mass into Kel, one word m per node pair (the block is m I for any nf); lumped mass, mass diagonal or mass action into Rel
 enum MassWhat { MASS_MATRIX = 1, MASS_LUMPED = 2, MASS_DIAG = 3, MASS_ACTION = 4 };
 
 struct ElementArgs {
@@ -184,6 +184,9 @@ struct ReduceArgs {
   double* R;                // full NF x NN field, or nullptr
 };
 int launch_reduce(int nf, const ReduceArgs& a, hipStream_t s);
+// CSR values of nf > 1 fields from element storage of one word per node pair, the blocks m I (mass matrices); kel_off:
+// the one-field table
+int launch_reduce_expand(int nf, const ReduceArgs& a, hipStream_t s);
 constexpr int RED_MERGE_LIGHT = 8, RED_MERGE_HEAVY = 4;  // rows per work-group of the merged launch's two buckets
 
 // Allocation-free assembly (noalloc.hip): a file-scope device array of NOALLOC_SCRATCH_BYTES per GPU holds the

@@ -7,8 +7,9 @@
 // (test/mechanics/TestMechanicsCommon.jl:52-124, rho = props[1]; test/poisson/TestPoissonCommon.jl:18-41, rho = 1),
 // assembled by assemble_mass! / assemble_lumped_mass! / assemble_diagonal! / assemble_matrix_action!
 // (src/assemblers/Matrix.jl:1-10, LumpedMass.jl:29-58, Diagonal.jl:17-68, MatrixAction.jl:154-238).
-// The outputs use the element kernels' storage (element-private FP32 Rel / symmetric NF x NF pair blocks in Kel),
-// so the FP64 reductions of reduce.hip sum them into the field or the CSR values unchanged.
+// The outputs use the element kernels' storage (element-private FP32 Rel / symmetric pair blocks in Kel), so the FP64
+// reductions of reduce.hip sum them into the field or the CSR values. The consistent mass has blocks m_ab I for any
+// number of fields: one word m_ab per pair is stored and the reduction writes the blocks out (reduce_expand_kernel).
 #include "fem_device.h"
 
 namespace fecx {
@@ -22,7 +23,8 @@ struct MassLDS {
     float w;
     float N[T::NNPE];
   };
-  static constexpr int KW = WHAT == MASS_MATRIX ? T::NPAIRS * NF * NF : 1;
+  static_assert(WHAT != MASS_MATRIX || NF == 1, "one word per node pair");
+  static constexpr int KW = WHAT == MASS_MATRIX ? T::NPAIRS : 1;
 };
 
 constexpr int MASS_THREADS = 256;
@@ -147,7 +149,7 @@ __global__ __launch_bounds__(256) void mass_kernel(ElementArgs args, float rho) 
     }
   }
   if constexpr (WHAT == MASS_MATRIX) {
-    // stage the blocks m_ab I in LDS over the consumed quadrature data, then copy each wavefront's contiguous range
+    // stage the words m_ab in LDS over the consumed quadrature data, then copy each wavefront's contiguous range
     // of element storage with consecutive lanes on consecutive words (the element kernels' store)
     __syncthreads();
     if (valid && lane < NNPE) {
@@ -157,13 +159,11 @@ __global__ __launch_bounds__(256) void mass_kernel(ElementArgs args, float rho) 
       for (int p = 0; p < MAXP; ++p)
         if (p < cnt) {
           const int b = lane + p < NNPE ? lane + p : lane + p - NNPE;
-          float* blk = dst + pair_pos(NNPE, lane, b, pair_lane_off(NNPE, lane) + p) * (NF * NF);
-#pragma unroll
-          for (int c = 0; c < NF * NF; ++c) blk[c] = (c % (NF + 1) == 0) ? kreg[p] : 0.0f;
+          dst[pair_pos(NNPE, lane, b, pair_lane_off(NNPE, lane) + p)] = kreg[p];
         }
     }
     __syncthreads();
-    constexpr int EW = T::NPAIRS * NF * NF;
+    constexpr int EW = T::NPAIRS;
     constexpr int EPWAVE = 64 / G;
     const int wl = threadIdx.x % 64, wv = threadIdx.x / 64;
     const int64_t e0 = args.ebeg + (int64_t)blockIdx.x * EPW + wv * EPWAVE;
@@ -192,7 +192,7 @@ static void launch_mass_kind(int what, const ElementArgs& a, float rho, hipStrea
   if (a.ne <= a.ebeg) return;
   const unsigned grid = (unsigned)((a.ne - a.ebeg + EPW - 1) / EPW);
   switch (what) {
-    case MASS_MATRIX: mass_kernel<KIND, NF, MASS_MATRIX><<<grid, MASS_THREADS, 0, s>>>(a, rho); break;
+    case MASS_MATRIX: mass_kernel<KIND, 1, MASS_MATRIX><<<grid, MASS_THREADS, 0, s>>>(a, rho); break;
     case MASS_LUMPED: mass_kernel<KIND, NF, MASS_LUMPED><<<grid, MASS_THREADS, 0, s>>>(a, rho); break;
     case MASS_DIAG: mass_kernel<KIND, NF, MASS_DIAG><<<grid, MASS_THREADS, 0, s>>>(a, rho); break;
     case MASS_ACTION: mass_kernel<KIND, NF, MASS_ACTION><<<grid, MASS_THREADS, 0, s>>>(a, rho); break;

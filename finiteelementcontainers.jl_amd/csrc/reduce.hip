@@ -16,6 +16,7 @@
 //                               reduce_scatter_kernel in one launch, their work-groups interleaved along the Morton curve;
 //   reduce_rows_kernel          slot-owner lanes for everything else: light scalar tet10/quad4 rows, 3-field light
 //                               rows of more than 32 blocks, heavy hex8/quad4 rows and tet10 rows of more than 72;
+//   reduce_expand_kernel        mass matrices of 2 or 3 fields, from one word per node pair (blocks m I);
 //   reduce_vector_kernel / reduce_vector_group_kernel   calls without CSR values (one thread, or 16 lanes, per row).
 // All sum a slot's (or a row's) contributions in ascending incidence order, so every form gives the same bits.
 #include <algorithm>
@@ -323,7 +324,7 @@ struct ScatterLDS {
   // lanes' registers instead
   static constexpr bool STAGE_R = LPR < 64;
   float s_r[STAGE_R ? NPW : 1][STAGE_R ? CHK : 1][NF];
-  double s_acc[NPW][SMAX * NB];
+  double s_acc[NPW][SMAX * NB + (LPR < 32 ? 1 : 0)];  // + 1: the rows that one LDS access spans start on different banks
 };
 // A row's lanes lie in one wavefront and share LDS with no other row: between its staging and its sums, ordering
 // comes from the program order of the wavefront's LDS operations, which complete in order, kept by a wavefront-scope
@@ -332,8 +333,9 @@ __device__ __forceinline__ void row_sync() {
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   __builtin_amdgcn_wave_barrier();
 }
-// The work-group's rows are the processing positions first + (thread / LPR), those below `end`.
-template <int NF, int NNPE, int LPR, int CHK, int SMAX>
+// The work-group's rows are the processing positions first + (thread / LPR), those below `end`. NFO > NF = 1: the blocks
+// are m I of NFO fields, m the stored word (reduce_expand_kernel).
+template <int NF, int NNPE, int LPR, int CHK, int SMAX, int NFO = NF>
 __device__ __forceinline__ void scatter_rows(const ReduceArgs& a, int64_t first, int64_t end, bool onepass,
                                              ScatterLDS<NF, NNPE, LPR, CHK, SMAX>& L) {
   static_assert(LPR <= 64 && 64 % LPR == 0, "a row's lanes lie in one wavefront");
@@ -453,6 +455,30 @@ __device__ __forceinline__ void scatter_rows(const ReduceArgs& a, int64_t first,
   }
   if (valid && a.R && lane < NF) a.R[n * NF + lane] = racc;
   // one wavefront wrote this row's accumulators, in order: no barrier before reading them back
+  if constexpr (NFO > NF) {
+    // the wavefront writes its rows one after the other, 64 consecutive values per store from a 128-byte boundary on, so
+    // that only a row's first and last line are written in part (185 us for the elastic hex8 64^3 mass against 214 with
+    // the stores starting at the row's first value)
+    static_assert(NF == 1, "expansion of scalar rows");
+    constexpr int RPW = 64 / LPR;  // rows per wavefront
+    const int wl = threadIdx.x % 64, g0 = threadIdx.x / 64 * RPW;
+#pragma unroll
+    for (int rr = 0; rr < RPW; ++rr) {
+      const int w = NFO * __builtin_amdgcn_readlane(deg, rr * LPR);  // values per CSR row of the node
+      double* dst = a.vals + (int64_t)(NFO * NFO) * __builtin_amdgcn_readlane(ri.z, rr * LPR);
+      const int before = (int)((reinterpret_cast<uintptr_t>(dst) >> 3) & 15);
+      for (int m = wl - before; m < NFO * w; m += 64) {
+        if (m < 0) continue;
+        int i = 0, c = m;  // row and column: m = i w + c
+#pragma unroll
+        for (int q = 1; q < NFO; ++q)
+          if (m >= q * w) { i = q; c = m - q * w; }
+        const int sl = c / NFO;
+        __builtin_nontemporal_store(c - sl * NFO == i ? s_acc[g0 + rr][sl] : 0.0, dst + m);
+      }
+    }
+    return;
+  }
   const int64_t rb = ri.z;
 #pragma unroll
   for (int i = 0; i < NF; ++i) {
@@ -470,6 +496,39 @@ __global__ __launch_bounds__(RED_THREADS) void reduce_scatter_kernel(ReduceArgs 
   __shared__ ScatterLDS<NF, NNPE, LPR, CHK, SMAX> L;
   constexpr int NPW = RED_THREADS / LPR;
   scatter_rows<NF, NNPE, LPR, CHK, SMAX>(a, a.p0 + xcd_chunk(blockIdx.x, gridDim.x) * NPW, a.p1, a.onepass != 0, L);
+}
+
+// Consistent mass of NFO fields: every block of an element matrix is m I, so the element kernel stores the one word m per
+// node pair (a ninth of the words of full 3 x 3 blocks) and the row's slots are summed as scalars and written out as
+// blocks, zeros included. Light rows take as many lanes as an element row has words (8, or 16 for tet10), heavier ones a
+// wavefront, with accumulators for the 255 blocks that a row may have. Elastic hex8 64^3 (65 million values): element
+// kernel and reduction 78 + 293 us with full blocks, 23 + 142 us with one word per pair.
+template <int NNPE, int NFO, int LPR, int CHK, int SMAX>
+__global__ __launch_bounds__(RED_THREADS) void reduce_expand_kernel(ReduceArgs a) {
+  __shared__ ScatterLDS<1, NNPE, LPR, CHK, SMAX> L;
+  constexpr int NPW = RED_THREADS / LPR;
+  scatter_rows<1, NNPE, LPR, CHK, SMAX, NFO>(a, a.p0 + xcd_chunk(blockIdx.x, gridDim.x) * NPW, a.p1, a.onepass != 0, L);
+}
+template <int NNPE, int NFO>
+static int launch_expand(const ReduceArgs& a, hipStream_t s) {
+  constexpr int LPR = NNPE == 10 ? 16 : 8;
+  ReduceArgs lo = a, hi = a;
+  lo.p1 = std::min(a.p1, a.nlight);
+  hi.p0 = std::max(a.p0, a.nlight);
+  lo.onepass = 1;
+  hi.onepass = 0;
+  auto grid = [](const ReduceArgs& r, int lpr) {  // the XCD remap needs a multiple of 8
+    return (unsigned)(((r.p1 - r.p0 + RED_THREADS / lpr - 1) / (RED_THREADS / lpr) + 7) / 8 * 8);
+  };
+  if (lo.p1 > lo.p0) {
+    if (a.maxdeg_light > 32) return -1;
+    reduce_expand_kernel<NNPE, NFO, LPR, CH, 32><<<grid(lo, LPR), RED_THREADS, 0, s>>>(lo);
+  }
+  if (hi.p1 > hi.p0) {
+    if (a.maxdeg > 256) return -1;
+    reduce_expand_kernel<NNPE, NFO, 64, RED_HEAVY_CH, 256><<<grid(hi, 64), RED_THREADS, 0, s>>>(hi);
+  }
+  return 0;
 }
 
 constexpr int HEAVY_SCATTER_SMAX = 72;  // structured tet10 vertex rows: 65 blocks
@@ -683,6 +742,14 @@ __global__ __launch_bounds__(256) void reduce_vector_group_kernel(ReduceArgs a) 
     if (pass + 1 < maxpass) __syncthreads();
   }
   if (valid && lane < NF) a.R[(int64_t)ri.x * NF + lane] = acc;
+}
+
+int launch_reduce_expand(int nf, const ReduceArgs& a, hipStream_t s) {
+  if (a.p1 <= a.p0 || !a.vals) return 0;
+  if (nf == 2 && a.nnpe == 4) return launch_expand<4, 2>(a, s);
+  if (nf == 3 && a.nnpe == 8) return launch_expand<8, 3>(a, s);
+  if (nf == 3 && a.nnpe == 10) return launch_expand<10, 3>(a, s);
+  return -1;
 }
 
 int launch_reduce(int nf, const ReduceArgs& a, hipStream_t s) {
