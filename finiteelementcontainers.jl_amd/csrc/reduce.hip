@@ -30,6 +30,16 @@ constexpr int CH = 8;            // incidences staged per pass
 constexpr int RED_NF1_LPR = 8;     // lanes per scalar row of at most 32 blocks
 constexpr int RED_NF3_LPR = 32;    // lanes per vector row of at most 32 blocks
 constexpr int RED_HEAVY_LPR = 128;  // lanes per row of 65..256 blocks (one slot per lane and sweep, two sweeps past 128)
+// Loads in flight per lane of the scatter: a divisor of the MAX loads of a pass. Three-field rows take 2 of a light row's 8
+// and 3 of a vertex row's 12 (neo-Hookean tet10 48^3 x 6 step: 1.334 ms; 1, 2 or 4 on both: 1.400, 1.341, 1.386; hex8 two
+// materials 43 x 37 x 51: 0.239-0.244 ms with 2 or 4); scalar rows, one word per load, as many as there are up to 4 (Poisson
+// tet10 28^3 x 6 step 134-137 us with 1 to 8).
+template <int NF, int MAX>
+constexpr int scatter_batch() {
+  int n = NF == 1 ? 4 : (MAX > 8 ? 3 : 2);
+  while (MAX % n) --n;
+  return n;
+}
 constexpr int RED_LB = 4;          // vector rows: incidences whose block loads are in flight together
 constexpr int RED_LB1 = 8;         // the same for rows with one staged word per lane and incidence
 constexpr int RED_HEAVY_CH = 24;   // incidences staged per pass on 128-lane rows (tet10 interior vertices: 24)
@@ -303,28 +313,41 @@ __global__ __launch_bounds__(RED_THREADS) void reduce_scalar_hex8_kernel(ReduceA
   for (int k = lane; k < deg; k += LPR) a.vals[(int64_t)ri.z + k] = s_acc[grp][k];
 }
 
-// Vector rows as a scatter, LPR lanes per row within one wavefront (light rows: 32 lanes, at most 8 incidences and 32
-// blocks; tet10 vertex rows: 64 lanes, 24 incidences per pass, 65 blocks). Lane l holds words l, l + LPR, ... of the
-// row's staged K_a* (block b = word / NF^2, entry c = word % NF^2) for each incidence, loaded a batch of incidences
-// at a time, and adds each into the FP64 accumulator of (slot of b, c) in LDS, incidence after incidence in ascending
-// order. Within one incidence the blocks land in distinct slots, and the LDS operations of one wavefront complete in
-// order, so every accumulator sums its words in the slot-owner kernel's order, with the same bits. The slot-owner
-// form tests every staged block's slot byte for every slot (240 tests per lane on a tet10 vertex row) and runs a
-// block's 9 FP64 adds on every lane whenever one lane matched: about 1,300 instructions per wavefront on the vertex
-// rows, which bound its time. Rows of more than SMAX blocks keep the slot-owner kernel.
+// Rows as a scatter, LPR lanes per row within one wavefront (light rows: at most 8 incidences and 32 blocks; tet10 vertex
+// rows: 64 lanes, 24 incidences per pass, 65 blocks). A lane holds one row (NF words, one load) of one block K_ab of an
+// incidence, loaded a batch of incidences at a time, and adds its words into the FP64 accumulators of the row's CSR values
+// in LDS, incidence after incidence in ascending order. Within one incidence the blocks land in distinct slots, and the LDS
+// operations of one wavefront complete in order, so every accumulator sums its words in the slot-owner kernel's order, with
+// the same bits. The slot-owner form tests every staged block's slot byte for every slot (240 tests per lane on a tet10
+// vertex row) and runs a block's 9 FP64 adds on every lane whenever one lane matched: about 1,300 instructions per wavefront
+// on the vertex rows, which bound its time. Rows of more than SMAX blocks keep the slot-owner kernel.
+//
+// What this form is bound by: instructions and address units rather than bytes, so it spends few of them. One lane per word
+// of K_a* (three loads, addresses and slot look-ups where there is now one) kept the VALU 67 % and the texture-address units
+// 72 % busy on tet10 48^3 x 6; a read-add-write per word made a chain of two LDS round trips of every word, where LDS
+// atomics without return (ds_add_f64) make nothing wait. An incidence's record and local node are decoded once, by the
+// lane that stages it. The accumulators lie in CSR order, so the row leaves as a copy, 64 consecutive values per store from
+// a 128-byte boundary on: only its first and last line are written in part (the lanes of a row storing each CSR row from its
+// first value on wrote 14 % more bytes). neo-Hookean tet10 48^3 x 6 reduction: 1.19 -> 0.95 ms
+// (3.9 GB at 4.1 TB/s, where a large copy moves 4.3 to 4.9).
+template <int NF, int NNPE, int LPR>
+struct ScatterShape {
+  static constexpr int ROWS = NNPE * NF;  // block rows of an incidence: one lane each
+  static constexpr int SUB = ROWS <= 8 ? 8 : (ROWS <= 16 ? 16 : 32);  // lanes per incidence
+  static constexpr int PH = LPR / SUB;    // incidences that a row's lanes hold at once
+  static_assert(ROWS <= SUB && LPR % SUB == 0, "an incidence's lanes lie in the row's");
+};
 template <int NF, int NNPE, int LPR, int CHK, int SMAX>
 struct ScatterLDS {
-  static constexpr int NPW = RED_THREADS / LPR, NB = NF * NF, VW = (NNPE + 3) / 4, BW = NNPE * NB;
-  // block (a, b) of the staged rows: first word of its block in the element storage, bit 15 set when the storage holds
-  // K_ba (the words then transposed); 2 * NNPE^2 bytes instead of 2 * NNPE * BW for a table of every word
+  static constexpr int NPW = RED_THREADS / LPR, NB = NF * NF, VW = (NNPE + 3) / 4;
+  // block (a, b) of the staged rows: first word of its block in the element storage, bit 15 set when the storage holds K_ba
   uint16_t s_blk[NNPE][NNPE];
-  int32_t s_v[NPW][CHK];
+  uint32_t s_e[NPW][CHK];       // first word of the incidence's element record
+  // slot of each local node's block, and, in a byte past them where there is one, the incidence's local node
   uint32_t s_w[NPW][CHK][VW];
-  // staged residual rows; 64-lane rows (one per wavefront, so a uniform incidence index) read them from the staging
-  // lanes' registers instead
-  static constexpr bool STAGE_R = LPR < 64;
-  float s_r[STAGE_R ? NPW : 1][STAGE_R ? CHK : 1][NF];
-  double s_acc[NPW][SMAX * NB + (LPR < 32 ? 1 : 0)];  // + 1: the rows that one LDS access spans start on different banks
+  static constexpr bool LA_IN_W = 4 * VW > NNPE;
+  uint8_t s_la[LA_IN_W ? 1 : NPW][LA_IN_W ? 4 : CHK];
+  double s_acc[NPW][SMAX * NB + (LPR < 32 ? 1 : 0)];  // + 1: the rows one LDS access spans start on different banks
 };
 // A row's lanes lie in one wavefront and share LDS with no other row: between its staging and its sums, ordering
 // comes from the program order of the wavefront's LDS operations, which complete in order, kept by a wavefront-scope
@@ -333,27 +356,25 @@ __device__ __forceinline__ void row_sync() {
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   __builtin_amdgcn_wave_barrier();
 }
-// The work-group's rows are the processing positions first + (thread / LPR), those below `end`. NFO > NF = 1: the blocks
-// are m I of NFO fields, m the stored word (reduce_expand_kernel).
+// The work-group's rows are the processing positions first + (thread / LPR), those below `end`; rows on fewer than 64
+// lanes have at most CHK incidences. NFO > NF = 1: the blocks are m I of NFO fields, m the stored word
+// (reduce_expand_kernel).
 template <int NF, int NNPE, int LPR, int CHK, int SMAX, int NFO = NF>
-__device__ __forceinline__ void scatter_rows(const ReduceArgs& a, int64_t first, int64_t end, bool onepass,
+__device__ __forceinline__ void scatter_rows(const ReduceArgs& a, int64_t first, int64_t end,
                                              ScatterLDS<NF, NNPE, LPR, CHK, SMAX>& L) {
   static_assert(LPR <= 64 && 64 % LPR == 0, "a row's lanes lie in one wavefront");
-  constexpr int NPW = RED_THREADS / LPR;
+  static_assert(NFO == NF || NF == 1, "expansion of scalar rows only");
+  using SH = ScatterShape<NF, NNPE, LPR>;
+  using LDS = ScatterLDS<NF, NNPE, LPR, CHK, SMAX>;
   constexpr int NB = NF * NF;                      // words per block
   constexpr int EW = NNPE * (NNPE + 1) / 2 * NB;   // stored words per element
   constexpr int VW = (NNPE + 3) / 4;               // vslot words per incidence
-  constexpr int BW = NNPE * NB;                    // staged words per incidence
-  constexpr int JN = (BW + LPR - 1) / LPR;         // words per lane and incidence
-  // incidences whose loads are in flight together: 2 on tet10 light rows (3 words per lane; neo-Hookean tet10 80^3 x 6
-  // reduction 5.72 against 5.85 ms with 4), 4 on hex8 ones (neo-Hookean hex8 96^3: 0.983 against 1.001 ms with 2)
-  constexpr int LB = JN <= 2 ? RED_LB1 : (NNPE == 10 ? 2 : RED_LB);
-  static_assert(CHK <= LPR && CHK % LB == 0, "a row's lanes stage its incidences, LB per batch");
+  constexpr int BW = NNPE * NB;                    // words of K_a*
+  constexpr int SUB = SH::SUB, PH = SH::PH;
+  constexpr int LB = scatter_batch<NF, CHK / PH>();  // loads in flight per lane
+  static_assert(CHK <= LPR && CHK % (LB * PH) == 0, "a row's lanes stage its incidences, LB PH per batch");
   auto& s_blk = L.s_blk;
-  auto& s_v = L.s_v;
   auto& s_w = L.s_w;
-  auto& s_r = L.s_r;
-  constexpr bool STAGE_R = ScatterLDS<NF, NNPE, LPR, CHK, SMAX>::STAGE_R;
   auto& s_acc = L.s_acc;
   for (int i = threadIdx.x; i < NNPE * NNPE; i += RED_THREADS) {  // from the word table: words 0 and 1 of each block
     const int16_t* o = a.kel_off + (i / NNPE) * BW + (i % NNPE) * NB;
@@ -368,45 +389,35 @@ __device__ __forceinline__ void scatter_rows(const ReduceArgs& a, int64_t first,
   const int32_t c0 = ri.y, ninc = ri.w & 0xFFFF;
   const int deg = a.vals ? (ri.w >> 16) : 0;  // 0: no CSR blocks (a node with Dirichlet dofs)
   for (int k = lane; k < deg * NB; k += LPR) s_acc[grp][k] = 0.0;
-  // passes of this row (light rows, at most CHK incidences, take one); the two rows of a 32-lane wavefront may differ
-  const int maxpass = onepass ? 1 : (ninc + CHK - 1) / CHK;
   __syncthreads();  // s_blk, the work-group's only barrier
-  // this lane's words: block and entry of word jj * LPR + lane, and the entry's place in the transposed block
-  int wb[JN], wc[JN], wt[JN];
-#pragma unroll
-  for (int jj = 0; jj < JN; ++jj) {
-    const int j = jj * LPR + lane;
-    wb[jj] = j < BW ? j / NB : 0;
-    wc[jj] = j % NB;
-    wt[jj] = (wc[jj] % NF) * NF + wc[jj] / NF;
-  }
+  // this lane: row r of the block of local node b, of incidence h of a group of PH
+  const int h = lane / SUB, l = lane % SUB;
+  const bool on = l < SH::ROWS;
+  const int b = on ? l / NF : 0, r = l % NF;
+  const int wv = NF * deg;  // values per CSR row of the node
   double racc = 0.0;
+  float rr[NF] = {};  // this lane's incidence's residual row
+  const int maxpass = LPR == 64 ? (ninc + CHK - 1) / CHK : 1;
   for (int pass = 0; pass < maxpass; ++pass) {
     const int base = pass * CHK;
     const int cnt = min(CHK, ninc - base);  // may be <= 0 for this node
-    float rr[NF] = {};  // 64-lane rows: this lane's incidence's residual row
     if (lane < cnt) {
       const int64_t c = (int64_t)c0 + base + lane;
-      const int32_t v = a.vent[c];
-      s_v[grp][lane] = v;
+      const uint32_t v = (uint32_t)a.vent[c];
+      L.s_e[grp][lane] = v / NNPE * (uint32_t)EW;  // element storage is limited to 2^31 words
+      const uint32_t la = v % NNPE;
+      if constexpr (!LDS::LA_IN_W) L.s_la[grp][lane] = (uint8_t)la;
       const uint32_t* sl = reinterpret_cast<const uint32_t*>(a.vslot) + c * VW;
 #pragma unroll
-      for (int q = 0; q < VW; ++q) s_w[grp][lane][q] = sl[q];
+      for (int q = 0; q < VW; ++q)
+        s_w[grp][lane][q] = LDS::LA_IN_W && q == VW - 1 ? (sl[q] & 0x00FFFFFFu) | (la << 24) : sl[q];
       if (a.R) {
 #pragma unroll
-        for (int i = 0; i < NF; ++i) {
-          const float r = a.Rel[(int64_t)v * NF + i];
-          if constexpr (STAGE_R) s_r[grp][lane][i] = r;
-          else rr[i] = r;
-        }
+        for (int i = 0; i < NF; ++i) rr[i] = a.Rel[(int64_t)v * NF + i];
       }
     }
-    row_sync();  // s_v, s_w and s_r staged by the row's lanes
-    if constexpr (STAGE_R) {
-      if (a.R && lane < NF) {
-        for (int t = 0; t < cnt; ++t) racc += (double)s_r[grp][t][lane];
-      }
-    } else if (a.R) {
+    row_sync();  // s_e, s_w and s_la staged by the row's lanes
+    if (LPR == 64 && a.R) {
       for (int t = 0; t < cnt; ++t) {  // lane i < NF adds entry i of incidence t's row, held by lane t
         float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rr[0]), t));
 #pragma unroll
@@ -419,83 +430,85 @@ __device__ __forceinline__ void scatter_rows(const ReduceArgs& a, int64_t first,
     }
     if (deg > 0) {
 #pragma unroll
-      for (int t0 = 0; t0 < CHK; t0 += LB) {
+      for (int t0 = 0; t0 < CHK; t0 += LB * PH) {
         if (t0 >= cnt) break;
-        float w[LB][JN];  // all loads of the batch in flight together
+        float w[LB][NF];      // all loads of the batch in flight together
+        uint32_t at[LB], st[LB];  // the first word's accumulator and the stride to the next word's
+        bool add[LB];
 #pragma unroll
         for (int tt = 0; tt < LB; ++tt) {
-          const int t = t0 + tt;
-          const uint32_t v = (uint32_t)s_v[grp][t < cnt ? t : 0];
-          const uint32_t ebase = (v / NNPE) * (uint32_t)EW;  // element storage is limited to 2^31 words
-          const int la = (int)(v % NNPE);
+          const int t = t0 + tt * PH + h, ts = t < cnt ? t : 0;
+          const uint8_t* wb = reinterpret_cast<const uint8_t*>(s_w[grp][ts]);
+          const uint32_t e = s_blk[LDS::LA_IN_W ? wb[4 * VW - 1] : L.s_la[grp][ts]][b], sb = wb[b];
+          const float* p = a.Kel + (L.s_e[grp][ts] + (e & 0x7FFFu) + (uint32_t)(r * NF));
 #pragma unroll
-          for (int jj = 0; jj < JN; ++jj) {
-            const uint32_t e = s_blk[la][wb[jj]];
-            const uint32_t off = (e & 0x7FFFu) + (uint32_t)((e & 0x8000u) ? wt[jj] : wc[jj]);
-            w[tt][jj] = a.Kel[ebase + (jj * LPR + lane < BW ? off : 0u)];
-          }
+          for (int k = 0; k < NF; ++k) w[tt][k] = p[k];
+          // the stored row r is row r of K_ab, or its column r where the storage holds K_ba
+          const bool tr = (e & 0x8000u) != 0;
+          at[tt] = sb * NF + (uint32_t)(tr ? r : r * wv);
+          st[tt] = (uint32_t)(tr ? wv : 1);
+          add[tt] = on && t < cnt && sb != 0xFFu;
         }
 #pragma unroll
-        for (int tt = 0; tt < LB; ++tt) {
-          const int t = t0 + tt;
-          if (t < cnt) {
+        for (int tt = 0; tt < LB; ++tt)
 #pragma unroll
-            for (int jj = 0; jj < JN; ++jj) {
-              if (jj * LPR + lane < BW) {
-                const int b = wb[jj];
-                const uint32_t sb = (s_w[grp][t][b >> 2] >> (8 * (b & 3))) & 0xFFu;  // the block's slot in the row
-                if (sb != 0xFFu) s_acc[grp][sb * NB + wc[jj]] += (double)w[tt][jj];
-              }
+          for (int ph = 0; ph < PH; ++ph)  // the incidences of the group one after the other
+            if (add[tt] && (PH == 1 || h == ph)) {
+#pragma unroll
+              for (int k = 0; k < NF; ++k)
+                (void)__hip_atomic_fetch_add(&s_acc[grp][at[tt] + k * st[tt]], (double)w[tt][k], __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_WORKGROUP);
             }
-          }
-        }
       }
     }
-    row_sync();  // the next pass restages s_v, s_w and s_r
+    row_sync();  // the next pass restages s_e, s_w and s_la
   }
-  if (valid && a.R && lane < NF) a.R[n * NF + lane] = racc;
-  // one wavefront wrote this row's accumulators, in order: no barrier before reading them back
-  if constexpr (NFO > NF) {
-    // the wavefront writes its rows one after the other, 64 consecutive values per store from a 128-byte boundary on, so
-    // that only a row's first and last line are written in part (185 us for the elastic hex8 64^3 mass against 214 with
-    // the stores starting at the row's first value)
-    static_assert(NF == 1, "expansion of scalar rows");
-    constexpr int RPW = 64 / LPR;  // rows per wavefront
-    const int wl = threadIdx.x % 64, g0 = threadIdx.x / 64 * RPW;
+  // the wavefront writes its rows' values one row after the other (a node's NFO CSR rows are contiguous)
+  constexpr int RPW = 64 / LPR;  // rows per wavefront
+  const int wl = threadIdx.x % 64, g0 = threadIdx.x / 64 * RPW;
 #pragma unroll
-    for (int rr = 0; rr < RPW; ++rr) {
-      const int w = NFO * __builtin_amdgcn_readlane(deg, rr * LPR);  // values per CSR row of the node
-      double* dst = a.vals + (int64_t)(NFO * NFO) * __builtin_amdgcn_readlane(ri.z, rr * LPR);
-      const int before = (int)((reinterpret_cast<uintptr_t>(dst) >> 3) & 15);
-      for (int m = wl - before; m < NFO * w; m += 64) {
-        if (m < 0) continue;
-        int i = 0, c = m;  // row and column: m = i w + c
+  for (int rw = 0; rw < RPW; ++rw) {
+    const int w = NFO * __builtin_amdgcn_readlane(deg, rw * LPR);
+    double* dst = a.vals + (int64_t)(NFO * NFO) * __builtin_amdgcn_readlane(ri.z, rw * LPR);
+    const int before = (int)((reinterpret_cast<uintptr_t>(dst) >> 3) & 15);
+    for (int m = wl - before; m < NFO * w; m += 64) {
+      if (m < 0) continue;
+      double x;
+      if constexpr (NFO > NF) {
+        int i = 0, c = m;  // CSR row and column: m = i w + c
 #pragma unroll
         for (int q = 1; q < NFO; ++q)
           if (m >= q * w) { i = q; c = m - q * w; }
         const int sl = c / NFO;
-        __builtin_nontemporal_store(c - sl * NFO == i ? s_acc[g0 + rr][sl] : 0.0, dst + m);
+        x = c - sl * NFO == i ? s_acc[g0 + rw][sl] : 0.0;
+      } else {
+        x = s_acc[g0 + rw][m];
       }
-    }
-    return;
-  }
-  const int64_t rb = ri.z;
-#pragma unroll
-  for (int i = 0; i < NF; ++i) {
-    double* dst = a.vals + (int64_t)NB * rb + (int64_t)i * NF * deg;
-    for (int m = lane; m < NF * deg; m += LPR) {
-      const double x = s_acc[grp][(m / NF) * NB + i * NF + m % NF];
-      if constexpr (NF >= 3) __builtin_nontemporal_store(x, dst + m);  // written once, never read here
+      if constexpr (NFO >= 2) __builtin_nontemporal_store(x, dst + m);  // written once, never read here
       else dst[m] = x;
     }
   }
+  if (!a.R) return;
+  if constexpr (LPR < 64) {
+    // the row's residual: the staged element rows through the accumulators' space, now read, summed in ascending order
+    row_sync();
+    const int cnt = min(CHK, ninc);
+    if (lane < cnt) {
+#pragma unroll
+      for (int i = 0; i < NF; ++i) s_acc[grp][lane * NF + i] = (double)rr[i];
+    }
+    row_sync();
+    if (lane < NF)
+      for (int t = 0; t < cnt; ++t) racc += s_acc[grp][t * NF + lane];
+  }
+  if (valid && lane < NF) a.R[n * NF + lane] = racc;
 }
 
 template <int NF, int NNPE, int LPR, int CHK, int SMAX>
 __global__ __launch_bounds__(RED_THREADS) void reduce_scatter_kernel(ReduceArgs a) {
   __shared__ ScatterLDS<NF, NNPE, LPR, CHK, SMAX> L;
   constexpr int NPW = RED_THREADS / LPR;
-  scatter_rows<NF, NNPE, LPR, CHK, SMAX>(a, a.p0 + xcd_chunk(blockIdx.x, gridDim.x) * NPW, a.p1, a.onepass != 0, L);
+  scatter_rows<NF, NNPE, LPR, CHK, SMAX>(a, a.p0 + xcd_chunk(blockIdx.x, gridDim.x) * NPW, a.p1, L);
 }
 
 // Consistent mass of NFO fields: every block of an element matrix is m I, so the element kernel stores the one word m per
@@ -507,7 +520,7 @@ template <int NNPE, int NFO, int LPR, int CHK, int SMAX>
 __global__ __launch_bounds__(RED_THREADS) void reduce_expand_kernel(ReduceArgs a) {
   __shared__ ScatterLDS<1, NNPE, LPR, CHK, SMAX> L;
   constexpr int NPW = RED_THREADS / LPR;
-  scatter_rows<1, NNPE, LPR, CHK, SMAX, NFO>(a, a.p0 + xcd_chunk(blockIdx.x, gridDim.x) * NPW, a.p1, a.onepass != 0, L);
+  scatter_rows<1, NNPE, LPR, CHK, SMAX, NFO>(a, a.p0 + xcd_chunk(blockIdx.x, gridDim.x) * NPW, a.p1, L);
 }
 template <int NNPE, int NFO>
 static int launch_expand(const ReduceArgs& a, hipStream_t s) {
@@ -515,8 +528,6 @@ static int launch_expand(const ReduceArgs& a, hipStream_t s) {
   ReduceArgs lo = a, hi = a;
   lo.p1 = std::min(a.p1, a.nlight);
   hi.p0 = std::max(a.p0, a.nlight);
-  lo.onepass = 1;
-  hi.onepass = 0;
   auto grid = [](const ReduceArgs& r, int lpr) {  // the XCD remap needs a multiple of 8
     return (unsigned)(((r.p1 - r.p0 + RED_THREADS / lpr - 1) / (RED_THREADS / lpr) + 7) / 8 * 8);
   };
@@ -525,8 +536,8 @@ static int launch_expand(const ReduceArgs& a, hipStream_t s) {
     reduce_expand_kernel<NNPE, NFO, LPR, CH, 32><<<grid(lo, LPR), RED_THREADS, 0, s>>>(lo);
   }
   if (hi.p1 > hi.p0) {
-    if (a.maxdeg > 256) return -1;
-    reduce_expand_kernel<NNPE, NFO, 64, RED_HEAVY_CH, 256><<<grid(hi, 64), RED_THREADS, 0, s>>>(hi);
+    if (a.maxdeg > 255) return -1;
+    reduce_expand_kernel<NNPE, NFO, 64, RED_HEAVY_CH, 255><<<grid(hi, 64), RED_THREADS, 0, s>>>(hi);
   }
   return 0;
 }
@@ -551,8 +562,8 @@ __global__ __launch_bounds__(RED_THREADS) __attribute__((amdgpu_waves_per_eu(8, 
   const int64_t c = xcd_chunk(blockIdx.x, gridDim.x);
   if (c >= a.nmerged) return;  // the grid is rounded up to a multiple of 8
   const int2 ch = a.merged[c];
-  if (ch.y == 0) scatter_rows<3, 10, 32, CH, 32>(a, ch.x, a.nlight, false, L.lo);
-  else scatter_rows<3, 10, 64, RED_HEAVY_CH, MERGED_HEAVY_SMAX>(a, ch.x, a.p1, false, L.hi);
+  if (ch.y == 0) scatter_rows<3, 10, 32, CH, 32>(a, ch.x, a.nlight, L.lo);
+  else scatter_rows<3, 10, 64, RED_HEAVY_CH, MERGED_HEAVY_SMAX>(a, ch.x, a.p1, L.hi);
 }
 
 // One launch over processing positions [a.p0, a.p1) whose rows have at most `maxdeg` blocks. Lanes per row: 8 for
