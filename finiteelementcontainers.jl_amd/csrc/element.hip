@@ -931,7 +931,8 @@ union FusedWork {
   double stage[NODES * 27 * NB];
 };
 
-template <int NF, int PHYS, int SX, int SY>
+// PART: the values go to the dof-level CSR of a partial Dirichlet set (csr_row).
+template <int NF, int PHYS, int SX, int SY, bool PART>
 __global__ __launch_bounds__(8 * SX * SY) __attribute__((amdgpu_waves_per_eu(NF == 1 ? 4 : 2, 8)))
 void fused_hex8_kernel(ElementArgs args, FusedArgs f) {
   using TL = FusedTile<SX, SY>;
@@ -1153,10 +1154,21 @@ void fused_hex8_kernel(ElementArgs args, FusedArgs f) {
           double v[NCH];
 #pragma unroll
           for (int c = 0; c < NCH; ++c) v[c] = wl + 64 * c < o.y ? src[wl + 64 * c] : 0.0;
-          double* dst = f.vals + (int64_t)NB * o.x;
+          if constexpr (PART) {
+            const CsrRow row = csr_row(f.vals, f.rmap, o.x, NB);
 #pragma unroll
-          for (int c = 0; c < NCH; ++c)
-            if (wl + 64 * c < o.y) __builtin_nontemporal_store(v[c], dst + wl + 64 * c);
+            for (int c = 0; c < NCH; ++c) {
+              const int m = wl + 64 * c;
+              if (m >= o.y) continue;
+              if (!row.map) __builtin_nontemporal_store(v[c], row.vals + m);
+              else if (const int q = row.map[m]; q >= 0) row.vals[q] = v[c];
+            }
+          } else {
+            double* dst = f.vals + (int64_t)NB * o.x;
+#pragma unroll
+            for (int c = 0; c < NCH; ++c)
+              if (wl + 64 * c < o.y) __builtin_nontemporal_store(v[c], dst + wl + 64 * c);
+          }
         }
       }
       // no barrier here: element_eval's first barrier comes before its first write to the work area
@@ -1222,18 +1234,23 @@ void scatter_hex8_kernel(ElementArgs args, FusedArgs f, int colour) {
     const int2 info = f.nodeinfo[na];
     const uint32_t mask = (uint32_t)info.y;
     const int deg = __popc(mask);
+    const CsrRow row = csr_row(f.vals, f.rmap, info.x, NB);
     for (int b = 0; b < 8; ++b) {
       const int d = (off[b][2] - off[a][2] + 1) * 9 + (off[b][1] - off[a][1] + 1) * 3 + (off[b][0] - off[a][0] + 1);
       if (!((mask >> d) & 1u)) continue;
       const int slot = __popc(mask & ((1u << d) - 1u));
       const PairRef pr = pair_ref(8, a, b);
       const float* blk = work.K + grp * KW + pr.slot * NB;
-      double* dst = f.vals + (int64_t)NB * info.x + NF * slot;
 #pragma unroll
       for (int i = 0; i < NF; ++i)
 #pragma unroll
         for (int k = 0; k < NF; ++k) {
-          double* p = dst + (int64_t)i * NF * deg + k;
+          int m = i * NF * deg + NF * slot + k;
+          if (row.map) {
+            m = row.map[m];
+            if (m < 0) continue;
+          }
+          double* p = row.vals + m;
           const double v = (double)blk[pr.ab ? i * NF + k : k * NF + i];
           if (ATOMIC) atomicAdd(p, v);
           else *p += v;
@@ -1273,10 +1290,13 @@ int launch_scatter_hex8(int nf, int scatter, const ElementArgs& a, const FusedAr
 
 // One work-group per slot the device holds at once (the kernel's occupancy times the CU count), each with an equal
 // share of the (tile, plane) units.
-template <int NF, int PHYS>
+template <int NF, int PHYS, bool PART = false>
 static bool launch_fused(const ElementArgs& a, FusedArgs f, hipStream_t s) {
+  if constexpr (NF > 1 && !PART) {
+    if (f.rmap) return launch_fused<NF, PHYS, true>(a, f, s);
+  }
   using TL = FusedTile<FUSED_SX, FUSED_SY>;
-  auto kern = fused_hex8_kernel<NF, PHYS, FUSED_SX, FUSED_SY>;
+  auto kern = fused_hex8_kernel<NF, PHYS, FUSED_SX, FUSED_SY, PART>;
   static int slots = 0;  // per instantiation; the same on every gfx950 device
   if (slots == 0) {
     int dev = 0, cus = 0, per = 0;

@@ -94,6 +94,7 @@ fecx::ReduceArgs reduce_args(fecx_ctx* ctx) {
   r.kel_off = get<int16_t>(ctx, "kel_off");
   r.merged = ctx->merged_rows ? get<int2>(ctx, "rmerge") : nullptr;
   r.nmerged = (int64_t)(get_bytes(ctx, "rmerge") / sizeof(int2));
+  r.rmap = ctx->partial ? get<int32_t>(ctx, "rmap") : nullptr;
   r.Kel = get<float>(ctx, "Kel");
   r.Rel = get<float>(ctx, "Rel");
   return r;
@@ -134,7 +135,7 @@ bool detect_structured_hex8(fecx_ctx* ctx) {
   return true;
 }
 
-// Per node {first CSR block of its row, mask of the 27 neighbours (dx, dy, dz) present in the row}, bit
+// Per node {first CSR block of its row (with a partial Dirichlet set: its place in the dof-level CSR, row_place), mask of the 27 neighbours (dx, dy, dz) present in the row}, bit
 // (dz + 1) 9 + (dy + 1) 3 + (dx + 1): the neighbour exists and both nodes are free. Checked against the pattern's
 // row degrees; returns false (and the fused path stays off) on a mismatch.
 bool build_nodeinfo(fecx_ctx* ctx) {
@@ -153,7 +154,7 @@ bool build_nodeinfo(fecx_ctx* ctx) {
     }
     if ((int64_t)__builtin_popcount(mask) != hp.bptr[r + 1] - hp.bptr[r]) return false;
     if (hp.bptr[r] >= (int64_t(1) << 31)) return false;
-    info[2 * n] = (int32_t)hp.bptr[r];
+    info[2 * n] = ctx->partial ? ctx->row_place[n] : (int32_t)hp.bptr[r];
     info[2 * n + 1] = (int32_t)mask;
   }
   upload(ctx, "nodeinfo", info);
@@ -178,14 +179,6 @@ int scatter_path(fecx_ctx* ctx, int mode, bool surrogate, bool noalloc) {
   if ((ctx->scatter == FECX_SCATTER_ATOMIC || ctx->scatter == FECX_SCATTER_COLOURED) && direct_ok && !noalloc)
     return ctx->scatter;
   return FECX_SCATTER_TWO_PHASE;
-}
-
-// With a partial Dirichlet set: the dof-level CSR values out of the node-block values the kernels assembled
-// (stream-ordered after them).
-void compact_values(fecx_ctx* ctx, const double* full, double* out) {
-  if (!ctx->partial || !out || ctx->nnz == 0) return;
-  fecx::launch_gather_unknowns(ctx->nnz, get<int64_t>(ctx, "cmap"), full, out, ctx->stream);
-  HIPCHK(hipGetLastError());
 }
 
 // The numeric flag before a launch: cleared on the device only if the last read-back did not find it clear.
@@ -220,8 +213,6 @@ void assemble(fecx_ctx* ctx, int mode, const double* U, const double* V, double*
               bool noalloc = false) {
   check_ready(ctx);
   require(U != nullptr, FECX_ERR_ARG, "U is NULL");
-  double* const vals_out = vals;  // the caller's CSR; with a partial Dirichlet set the kernels fill vals_full
-  if (ctx->partial && vals) vals = get<double>(ctx, "vals_full");
   const bool surrogate_phys = ctx->mp.phys == FECX_J2_SURROGATE || ctx->mp.phys == FECX_NH_SURROGATE;
   const bool surrogate = surrogate_phys && ctx->sg_enabled;
   float *kel = get<float>(ctx, "Kel"), *rel = get<float>(ctx, "Rel");
@@ -266,6 +257,7 @@ void assemble(fecx_ctx* ctx, int mode, const double* U, const double* V, double*
     fa.nx = ctx->snx; fa.ny = ctx->sny; fa.nz = ctx->snz;
     fa.epos = get<int32_t>(ctx, "epos");
     fa.nodeinfo = get<int2>(ctx, "nodeinfo");
+    fa.rmap = ctx->partial ? get<int32_t>(ctx, "rmap") : nullptr;
     fa.vals = (mode & fecx::MODE_K) ? vals : nullptr;
     fa.R = (mode & fecx::MODE_R) ? R : nullptr;
     int rc = 0;
@@ -274,14 +266,13 @@ void assemble(fecx_ctx* ctx, int mode, const double* U, const double* V, double*
     } else {  // atomic or coloured: zero-fill, then every element adds its blocks and rows in place
       const size_t rbytes = sizeof(double) * (size_t)ctx->nn * ctx->nf;
       prof.run(path == FECX_SCATTER_ATOMIC ? "atomic" : "coloured", ctx->stream, [&] {
-        if (fa.vals) HIPCHK(hipMemsetAsync(fa.vals, 0, sizeof(double) * (size_t)ctx->nnz_full, ctx->stream));
+        if (fa.vals) HIPCHK(hipMemsetAsync(fa.vals, 0, sizeof(double) * (size_t)ctx->nnz, ctx->stream));
         if (fa.R) HIPCHK(hipMemsetAsync(fa.R, 0, rbytes, ctx->stream));
         rc = fecx::launch_scatter_hex8(ctx->nf, path == FECX_SCATTER_ATOMIC ? 1 : 2, ea, fa, ctx->stream);
       });
     }
     require(rc == 0, FECX_ERR_UNSUPPORTED, "no kernel of this scatter design for this nf / physics");
     HIPCHK(hipGetLastError());
-    compact_values(ctx, vals, vals_out);
     const int hflag = read_flag(ctx, flag);
     prof.finish();
     require(hflag == 0, FECX_ERR_NUMERIC, "element kernel met a non-positive Jacobian determinant or a NaN");
@@ -335,7 +326,6 @@ void assemble(fecx_ctx* ctx, int mode, const double* U, const double* V, double*
     require(rc == 0, FECX_ERR_UNSUPPORTED, "no reduction kernel for this element kind / nf");
     HIPCHK(hipGetLastError());
   }
-  compact_values(ctx, vals, vals_out);
   const int hflag = read_flag(ctx, flag);
   prof.finish();
   if (surrogate) fecx::surrogate_qp_finish(ctx);
@@ -358,7 +348,7 @@ void assemble_mass(fecx_ctx* ctx, int what, double density, const double* V, dou
   HIPCHK(hipGetLastError());
   fecx::ReduceArgs ra = reduce_args(ctx);
   ra.R = R;
-  ra.vals = (ctx->partial && vals) ? get<double>(ctx, "vals_full") : vals;
+  ra.vals = vals;
   const bool expand = what == fecx::MASS_MATRIX && ctx->nf > 1;  // one word per node pair: the blocks are m I
   if (expand) ra.kel_off = get<int16_t>(ctx, "kel_off1");
   prof.run("reduce", ctx->stream, [&] {
@@ -366,7 +356,6 @@ void assemble_mass(fecx_ctx* ctx, int what, double density, const double* V, dou
   });
   require(rc == 0, FECX_ERR_UNSUPPORTED, "no reduction kernel for this element kind / nf");
   HIPCHK(hipGetLastError());
-  compact_values(ctx, ra.vals, vals);
   const int hflag = read_flag(ctx, flag);
   prof.finish();
   require(hflag == 0, FECX_ERR_NUMERIC, "mass kernel met a non-positive Jacobian determinant");
@@ -537,11 +526,13 @@ int fecx_build_pattern(fecx_ctx* ctx, int64_t* nnz) {
       // rows and columns in ascending dof order, which is node-block order restricted to the unknown dofs
       std::vector<int64_t> ridx((size_t)ctx->nn * nf, -1);
       for (size_t i = 0; i < ctx->unknown_dofs.size(); ++i) ridx[ctx->unknown_dofs[i] - 1] = (int64_t)i;
-      std::vector<int64_t> cmap;
       ctx->red_of_full.assign((size_t)ctx->nnz_full, -1);
+      ctx->row_place.assign((size_t)ctx->nn, 0);
+      std::vector<int32_t> rmap;
       ctx->rptr.push_back(0);
       for (int64_t r = 0; r < hp.nfree; ++r) {
-        const int64_t n = hp.free_node[r], b0 = hp.bptr[r], deg = hp.bptr[r + 1] - b0;
+        const int64_t n = hp.free_node[r], b0 = hp.bptr[r], deg = hp.bptr[r + 1] - b0, full0 = (int64_t)nf * nf * b0;
+        const int64_t first = (int64_t)ctx->rcol.size();
         for (int i = 0; i < nf; ++i) {
           if (ridx[n * nf + i] < 0) continue;
           require(ridx[n * nf + i] == (int64_t)ctx->rptr.size() - 1, FECX_ERR_STATE, "unknown dof order");
@@ -549,23 +540,28 @@ int fecx_build_pattern(fecx_ctx* ctx, int64_t* nnz) {
             const int64_t m = hp.free_node[hp.bcol[b0 + sl]];
             for (int k = 0; k < nf; ++k) {
               if (ridx[m * nf + k] < 0) continue;
-              const int64_t full = (int64_t)nf * nf * b0 + (int64_t)i * nf * deg + (int64_t)nf * sl + k;
-              ctx->red_of_full[full] = (int64_t)cmap.size();
-              cmap.push_back(full);
+              ctx->red_of_full[full0 + (int64_t)i * nf * deg + (int64_t)nf * sl + k] = (int64_t)ctx->rcol.size();
               ctx->rcol.push_back(ridx[m * nf + k]);
             }
           }
           ctx->rptr.push_back((int64_t)ctx->rcol.size());
         }
+        require((int64_t)ctx->rcol.size() < (int64_t(1) << 31), FECX_ERR_UNSUPPORTED, "more than 2^31 - 1 CSR entries");
+        if ((int64_t)ctx->rcol.size() - first == (int64_t)nf * nf * deg) {
+          ctx->row_place[n] = (int32_t)first;
+        } else {
+          require((int64_t)rmap.size() + (int64_t)nf * nf * deg < (int64_t(1) << 31), FECX_ERR_UNSUPPORTED,
+                  "more than 2^31 - 1 mapped CSR entries");
+          ctx->row_place[n] = ~(int32_t)rmap.size();
+          for (int64_t e = 0; e < (int64_t)nf * nf * deg; ++e) rmap.push_back((int32_t)ctx->red_of_full[full0 + e]);
+        }
       }
       require((int64_t)ctx->rptr.size() == (int64_t)ctx->unknown_dofs.size() + 1, FECX_ERR_STATE, "row count");
-      ctx->nnz = (int64_t)cmap.size();
-      require(ctx->nnz < (int64_t(1) << 31), FECX_ERR_UNSUPPORTED, "more than 2^31 - 1 CSR entries");
+      ctx->nnz = (int64_t)ctx->rcol.size();
       std::vector<int32_t> rcol32(ctx->rcol.begin(), ctx->rcol.end());
-      upload(ctx, "cmap", cmap);
+      upload(ctx, "rmap", rmap);
       upload(ctx, "rptr", ctx->rptr);
       upload(ctx, "rcol", rcol32);
-      dev(ctx, "vals_full", sizeof(double) * (size_t)std::max<int64_t>(ctx->nnz_full, 1));
     }
     std::vector<int32_t> conn_s(ctx->ne * ctx->nnpe);  // connectivity in element storage order
     for (int64_t s = 0; s < ctx->ne; ++s)
@@ -598,7 +594,7 @@ int fecx_build_pattern(fecx_ctx* ctx, int64_t* nnz) {
         require(ninc < 65536, FECX_ERR_UNSUPPORTED, "a node has more than 65535 incident elements");
         ri[4 * p + 0] = n;
         ri[4 * p + 1] = pordered ? (int32_t)c : k0;
-        ri[4 * p + 2] = r >= 0 ? (int32_t)hp.bptr[r] : 0;
+        ri[4 * p + 2] = r < 0 ? 0 : (ctx->partial ? ctx->row_place[n] : (int32_t)hp.bptr[r]);
         ri[4 * p + 3] = ninc | (int32_t)(deg << 16);
         if (!pordered) continue;
         for (int32_t t = 0; t < ninc; ++t) {

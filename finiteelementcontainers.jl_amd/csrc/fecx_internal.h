@@ -113,6 +113,17 @@ __device__ __forceinline__ int64_t xcd_chunk(int64_t wg, int64_t nwg) {
   return (wg % 8) * per + wg / 8;
 }
 
+// A node's CSR values: entry m of its NB deg values goes to vals[m] or, map given, to vals[map[m]] unless that is -1 (a
+// fixed row or column of a partial Dirichlet set). place: first CSR block, or with rmap the row's row_place.
+struct CsrRow {
+  double* vals;
+  const int32_t* map;
+};
+__device__ __forceinline__ CsrRow csr_row(double* vals, const int32_t* rmap, int place, int nb) {
+  if (!rmap) return {vals + (int64_t)nb * place, nullptr};
+  return place >= 0 ? CsrRow{vals + place, nullptr} : CsrRow{vals, rmap + ~place};
+}
+
 struct MatParams {
   int phys;
   int source_kind;
@@ -151,9 +162,10 @@ struct FusedArgs {
   int nx, ny, nz;                // node counts per direction
   int tiles_x, tiles_y;          // node tiles per direction (set by launch_fused_hex8)
   const int32_t* epos;           // element id -> storage position
-  const int2* nodeinfo;          // per node: {first CSR block of its row, mask of the 27 neighbours in the row}
+  const int2* nodeinfo;          // per node: {first CSR block of its row, or row_place; mask of the 27 neighbours in the row}
   double* vals;                  // CSR values (or nullptr)
   double* R;                     // full NF x NN residual field (or nullptr)
+  const int32_t* rmap;           // dof-level CSR of a partial Dirichlet set: positions of its rows' entries; else nullptr
 };
 // returns 0, or -1 if the (nf, phys) combination has no fused kernel (or the mesh exceeds 2^31 tile planes)
 int launch_fused_hex8(int nf, const ElementArgs& a, const FusedArgs& f, hipStream_t s);
@@ -169,7 +181,9 @@ struct ReduceArgs {
   int onepass;              // every row of this launch has at most CH incidences (one pass, no pass-count vote)
   int64_t npad;             // positions [0, npad) hold padded rows: incidence slots vent[8 p .. 8 p + 7]
   int padded;               // this launch reads the padded slots directly (every row of it is padded)
-  const int4* rowinfo;      // per processing position: {node, first incidence slot, first CSR block or 0, ninc | degree << 16}
+  // per processing position: {node, first incidence slot, first CSR block (with rmap: row_place) or 0, ninc | degree << 16}
+  const int4* rowinfo;
+  const int32_t* rmap;      // dof-level CSR of a partial Dirichlet set: positions of its rows' entries; else nullptr
   int nnpe, maxdeg;
   const int32_t* vent;
   const uint8_t* vslot;
@@ -245,11 +259,14 @@ struct fecx_ctx {
   fecx::HostPattern hp;
   int64_t nnz = 0;       // entries of the CSR the caller sees
   int64_t nnz_full = 0;  // entries of the node-block layout the kernels assemble (NF^2 per block)
-  // a Dirichlet set that constrains some but not all dofs of a node (nf > 1, not condensed): the kernels assemble the
-  // node-block pattern of the nodes with a free dof into "vals_full", and a gather through "cmap" forms the reference's
-  // dof-level CSR (rows and columns of the unknown dofs); rptr/rcol are that CSR (0-based), red_of_full its inverse map
+  // a Dirichlet set that constrains some but not all dofs of a node (nf > 1, not condensed): the kernels sum the
+  // node-block pattern of the nodes with a free dof and write the reference's dof-level CSR (rows and columns of the
+  // unknown dofs); rptr/rcol are that CSR (0-based), red_of_full the position of every node-block entry in it or -1.
+  // row_place: per node, where its NF^2 deg values start in it (they are contiguous there unless a dof of the node or of a
+  // column is fixed), or, for such a row, the complement of its first entry in the device list "rmap" of positions
   bool partial = false;
   std::vector<int64_t> rptr, rcol, red_of_full;
+  std::vector<int32_t> row_place;
   // material: one per element block (foreach_block's per-block physics and properties); mp is block 0's
   bool has_material = false;
   fecx::MatParams mp{};

@@ -20,6 +20,7 @@
 //   reduce_vector_kernel / reduce_vector_group_kernel   calls without CSR values (one thread, or 16 lanes, per row).
 // All sum a slot's (or a row's) contributions in ascending incidence order, so every form gives the same bits.
 #include <algorithm>
+#include <type_traits>
 
 #include "fecx_internal.h"
 
@@ -118,7 +119,6 @@ void reduce_rows_kernel(ReduceArgs a) {
   // a row of a node with Dirichlet dofs has no CSR blocks (degree 0); a free node always couples with itself
   const int deg = a.vals ? (ri.w >> 16) : 0;
   const int32_t r = deg > 0 ? 0 : -1;
-  const int64_t rb = ri.z;
   double acc[SW][NF * NF];
 #pragma unroll
   for (int t = 0; t < SW; ++t)
@@ -232,16 +232,21 @@ void reduce_rows_kernel(ReduceArgs a) {
   }
   if (valid && a.R && lane < NF) a.R[n * NF + lane] = racc;
   if (r >= 0) {
+    const CsrRow row = csr_row(a.vals, NF > 1 ? a.rmap : nullptr, ri.z, NF * NF);
 #pragma unroll
     for (int sw = 0; sw < SW; ++sw) {
       const int s = lane + sw * LPR;
       if (s < deg) {
-        const int64_t base = (int64_t)NF * NF * rb + (int64_t)NF * s;
 #pragma unroll
         for (int i = 0; i < NF; ++i)
 #pragma unroll
           for (int k = 0; k < NF; ++k) {
-            double* dst = &a.vals[base + (int64_t)i * NF * deg + k];
+            int m = (i * deg + s) * NF + k;
+            if (NF > 1 && row.map) {
+              m = row.map[m];
+              if (m < 0) continue;
+            }
+            double* dst = row.vals + m;
             if constexpr (NF >= 3) __builtin_nontemporal_store(acc[sw][i * NF + k], dst);  // written once, never read here
             else *dst = acc[sw][i * NF + k];
           }
@@ -359,7 +364,9 @@ __device__ __forceinline__ void row_sync() {
 // The work-group's rows are the processing positions first + (thread / LPR), those below `end`; rows on fewer than 64
 // lanes have at most CHK incidences. NFO > NF = 1: the blocks are m I of NFO fields, m the stored word
 // (reduce_expand_kernel).
-template <int NF, int NNPE, int LPR, int CHK, int SMAX, int NFO = NF>
+// PART: the values go to the dof-level CSR of a partial Dirichlet set (csr_row); a compile-time choice, since the test in the
+// store loop cost the tet10 reduction 5 % and the fused hex8 kernel 3 %.
+template <bool PART, int NF, int NNPE, int LPR, int CHK, int SMAX, int NFO = NF>
 __device__ __forceinline__ void scatter_rows(const ReduceArgs& a, int64_t first, int64_t end,
                                              ScatterLDS<NF, NNPE, LPR, CHK, SMAX>& L) {
   static_assert(LPR <= 64 && 64 % LPR == 0, "a row's lanes lie in one wavefront");
@@ -469,8 +476,9 @@ __device__ __forceinline__ void scatter_rows(const ReduceArgs& a, int64_t first,
 #pragma unroll
   for (int rw = 0; rw < RPW; ++rw) {
     const int w = NFO * __builtin_amdgcn_readlane(deg, rw * LPR);
-    double* dst = a.vals + (int64_t)(NFO * NFO) * __builtin_amdgcn_readlane(ri.z, rw * LPR);
-    const int before = (int)((reinterpret_cast<uintptr_t>(dst) >> 3) & 15);
+    const CsrRow row = csr_row(a.vals, PART ? a.rmap : nullptr, __builtin_amdgcn_readlane(ri.z, rw * LPR), NFO * NFO);
+    double* dst = row.vals;
+    const int before = PART && row.map ? 0 : (int)((reinterpret_cast<uintptr_t>(dst) >> 3) & 15);
     for (int m = wl - before; m < NFO * w; m += 64) {
       if (m < 0) continue;
       double x;
@@ -484,8 +492,12 @@ __device__ __forceinline__ void scatter_rows(const ReduceArgs& a, int64_t first,
       } else {
         x = s_acc[g0 + rw][m];
       }
-      if constexpr (NFO >= 2) __builtin_nontemporal_store(x, dst + m);  // written once, never read here
-      else dst[m] = x;
+      if constexpr (NFO >= 2) {
+        if (!PART || !row.map) __builtin_nontemporal_store(x, dst + m);  // written once, never read here
+        else if (const int q = row.map[m]; q >= 0) dst[q] = x;
+      } else {
+        dst[m] = x;
+      }
     }
   }
   if (!a.R) return;
@@ -504,11 +516,11 @@ __device__ __forceinline__ void scatter_rows(const ReduceArgs& a, int64_t first,
   if (valid && lane < NF) a.R[n * NF + lane] = racc;
 }
 
-template <int NF, int NNPE, int LPR, int CHK, int SMAX>
+template <bool PART, int NF, int NNPE, int LPR, int CHK, int SMAX>
 __global__ __launch_bounds__(RED_THREADS) void reduce_scatter_kernel(ReduceArgs a) {
   __shared__ ScatterLDS<NF, NNPE, LPR, CHK, SMAX> L;
   constexpr int NPW = RED_THREADS / LPR;
-  scatter_rows<NF, NNPE, LPR, CHK, SMAX>(a, a.p0 + xcd_chunk(blockIdx.x, gridDim.x) * NPW, a.p1, L);
+  scatter_rows<PART, NF, NNPE, LPR, CHK, SMAX>(a, a.p0 + xcd_chunk(blockIdx.x, gridDim.x) * NPW, a.p1, L);
 }
 
 // Consistent mass of NFO fields: every block of an element matrix is m I, so the element kernel stores the one word m per
@@ -516,13 +528,13 @@ __global__ __launch_bounds__(RED_THREADS) void reduce_scatter_kernel(ReduceArgs 
 // blocks, zeros included. Light rows take as many lanes as an element row has words (8, or 16 for tet10), heavier ones a
 // wavefront, with accumulators for the 255 blocks that a row may have. Elastic hex8 64^3 (65 million values): element
 // kernel and reduction 78 + 293 us with full blocks, 23 + 142 us with one word per pair.
-template <int NNPE, int NFO, int LPR, int CHK, int SMAX>
+template <bool PART, int NNPE, int NFO, int LPR, int CHK, int SMAX>
 __global__ __launch_bounds__(RED_THREADS) void reduce_expand_kernel(ReduceArgs a) {
   __shared__ ScatterLDS<1, NNPE, LPR, CHK, SMAX> L;
   constexpr int NPW = RED_THREADS / LPR;
-  scatter_rows<1, NNPE, LPR, CHK, SMAX, NFO>(a, a.p0 + xcd_chunk(blockIdx.x, gridDim.x) * NPW, a.p1, L);
+  scatter_rows<PART, 1, NNPE, LPR, CHK, SMAX, NFO>(a, a.p0 + xcd_chunk(blockIdx.x, gridDim.x) * NPW, a.p1, L);
 }
-template <int NNPE, int NFO>
+template <bool PART, int NNPE, int NFO>
 static int launch_expand(const ReduceArgs& a, hipStream_t s) {
   constexpr int LPR = NNPE == 10 ? 16 : 8;
   ReduceArgs lo = a, hi = a;
@@ -533,11 +545,11 @@ static int launch_expand(const ReduceArgs& a, hipStream_t s) {
   };
   if (lo.p1 > lo.p0) {
     if (a.maxdeg_light > 32) return -1;
-    reduce_expand_kernel<NNPE, NFO, LPR, CH, 32><<<grid(lo, LPR), RED_THREADS, 0, s>>>(lo);
+    reduce_expand_kernel<PART, NNPE, NFO, LPR, CH, 32><<<grid(lo, LPR), RED_THREADS, 0, s>>>(lo);
   }
   if (hi.p1 > hi.p0) {
     if (a.maxdeg > 255) return -1;
-    reduce_expand_kernel<NNPE, NFO, 64, RED_HEAVY_CH, 255><<<grid(hi, 64), RED_THREADS, 0, s>>>(hi);
+    reduce_expand_kernel<PART, NNPE, NFO, 64, RED_HEAVY_CH, 255><<<grid(hi, 64), RED_THREADS, 0, s>>>(hi);
   }
   return 0;
 }
@@ -551,6 +563,7 @@ constexpr int MERGED_HEAVY_SMAX = 65;   // the same rows in reduce_merged_kernel
 // own launch reads the blocks its rows share with the other bucket's rows (24 of an element's 55) a second time,
 // long after the first; here the vertex and edge rows of the same elements run at about the same time on the same
 // XCD. Every row's sums are those of the bucket kernels, so the bits are too.
+template <bool PART>
 __global__ __launch_bounds__(RED_THREADS) __attribute__((amdgpu_waves_per_eu(8, 8))) void reduce_merged_kernel(
     ReduceArgs a) {
   static_assert(RED_THREADS / 32 == RED_MERGE_LIGHT && RED_THREADS / 64 == RED_MERGE_HEAVY, "chunk sizes");
@@ -562,8 +575,8 @@ __global__ __launch_bounds__(RED_THREADS) __attribute__((amdgpu_waves_per_eu(8, 
   const int64_t c = xcd_chunk(blockIdx.x, gridDim.x);
   if (c >= a.nmerged) return;  // the grid is rounded up to a multiple of 8
   const int2 ch = a.merged[c];
-  if (ch.y == 0) scatter_rows<3, 10, 32, CH, 32>(a, ch.x, a.nlight, L.lo);
-  else scatter_rows<3, 10, 64, RED_HEAVY_CH, MERGED_HEAVY_SMAX>(a, ch.x, a.p1, L.hi);
+  if (ch.y == 0) scatter_rows<PART, 3, 10, 32, CH, 32>(a, ch.x, a.nlight, L.lo);
+  else scatter_rows<PART, 3, 10, 64, RED_HEAVY_CH, MERGED_HEAVY_SMAX>(a, ch.x, a.p1, L.hi);
 }
 
 // One launch over processing positions [a.p0, a.p1) whose rows have at most `maxdeg` blocks. Lanes per row: 8 for
@@ -632,13 +645,15 @@ static int launch_buckets(const ReduceArgs& a, hipStream_t s) {
     if (NNPE == 10 && a.merged && a.nmerged > 0 && a.p0 == 0 && a.nlight < a.p1 && a.maxdeg_light <= 32 &&
         a.maxdeg <= MERGED_HEAVY_SMAX) {
       const int64_t grid = (a.nmerged + 7) / 8 * 8;  // XCD remap needs a multiple of 8
-      reduce_merged_kernel<<<(unsigned)grid, RED_THREADS, 0, s>>>(a);
+      if (a.rmap) reduce_merged_kernel<true><<<(unsigned)grid, RED_THREADS, 0, s>>>(a);
+      else reduce_merged_kernel<false><<<(unsigned)grid, RED_THREADS, 0, s>>>(a);
       return 0;
     }
     if (lo.p1 > lo.p0 && a.maxdeg_light <= 32) {
       int64_t grid = (lo.p1 - lo.p0 + RED_THREADS / 32 - 1) / (RED_THREADS / 32);
       grid = (grid + 7) / 8 * 8;  // XCD remap needs a multiple of 8
-      reduce_scatter_kernel<NF, NNPE, 32, CH, 32><<<(unsigned)grid, RED_THREADS, 0, s>>>(lo);
+      if (a.rmap) reduce_scatter_kernel<true, NF, NNPE, 32, CH, 32><<<(unsigned)grid, RED_THREADS, 0, s>>>(lo);
+      else reduce_scatter_kernel<false, NF, NNPE, 32, CH, 32><<<(unsigned)grid, RED_THREADS, 0, s>>>(lo);
     } else {
       rc = launch_lpr<NF, NNPE>(lo, a.maxdeg_light, s);
     }
@@ -650,7 +665,9 @@ static int launch_buckets(const ReduceArgs& a, hipStream_t s) {
     if (a.maxdeg <= HEAVY_SCATTER_SMAX) {
       int64_t grid = (hi.p1 - hi.p0 + RED_THREADS / 64 - 1) / (RED_THREADS / 64);
       grid = (grid + 7) / 8 * 8;  // XCD remap needs a multiple of 8
-      reduce_scatter_kernel<NF, NNPE, 64, RED_HEAVY_CH, HEAVY_SCATTER_SMAX><<<(unsigned)grid, RED_THREADS, 0, s>>>(hi);
+      constexpr int SM = HEAVY_SCATTER_SMAX;
+      if (NF > 1 && a.rmap) reduce_scatter_kernel<NF != 1, NF, NNPE, 64, RED_HEAVY_CH, SM><<<(unsigned)grid, RED_THREADS, 0, s>>>(hi);
+      else reduce_scatter_kernel<false, NF, NNPE, 64, RED_HEAVY_CH, SM><<<(unsigned)grid, RED_THREADS, 0, s>>>(hi);
       return 0;
     }
   }
@@ -757,10 +774,14 @@ __global__ __launch_bounds__(256) void reduce_vector_group_kernel(ReduceArgs a) 
 
 int launch_reduce_expand(int nf, const ReduceArgs& a, hipStream_t s) {
   if (a.p1 <= a.p0 || !a.vals) return 0;
-  if (nf == 2 && a.nnpe == 4) return launch_expand<4, 2>(a, s);
-  if (nf == 3 && a.nnpe == 8) return launch_expand<8, 3>(a, s);
-  if (nf == 3 && a.nnpe == 10) return launch_expand<10, 3>(a, s);
-  return -1;
+  auto go = [&](auto part) {
+    constexpr bool PART = decltype(part)::value;
+    if (nf == 2 && a.nnpe == 4) return launch_expand<PART, 4, 2>(a, s);
+    if (nf == 3 && a.nnpe == 8) return launch_expand<PART, 8, 3>(a, s);
+    if (nf == 3 && a.nnpe == 10) return launch_expand<PART, 10, 3>(a, s);
+    return -1;
+  };
+  return a.rmap ? go(std::true_type()) : go(std::false_type());
 }
 
 int launch_reduce(int nf, const ReduceArgs& a, hipStream_t s) {
