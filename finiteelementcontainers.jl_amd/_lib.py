@@ -58,6 +58,7 @@ _SIGS = {
     "fecx_assemble_mass_action": [ctypes.c_void_p, ctypes.c_double, ctypes.c_void_p, ctypes.c_void_p],
     "fecx_update_field_unknowns": [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
     "fecx_update_field_dirichlet": [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
+    "fecx_update_fields": [ctypes.c_void_p] * 6,
     "fecx_extract_field_unknowns": [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
     "fecx_csr_spmv": [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],
     "fecx_csr_diagonal_inverse": [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p],

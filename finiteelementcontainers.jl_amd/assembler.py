@@ -485,11 +485,9 @@ def create_parameters(mesh, asm, physics, props=None, dirichlet_bcs=(), times=(0
 
 def _update_for_assembly(p, asm, Uu, Vu=None):
     """_update_for_assembly! (src/Parameters.jl:404-425): BC values, then unknowns, into the full fields."""
-    if len(asm.dof.dirichlet_dofs):
-        asm.ctx.call("fecx_update_field_dirichlet", _ptr(p._bc_vals), _ptr(p.field))
-    asm.ctx.call("fecx_update_field_unknowns", _ptr(Uu), _ptr(p.field))
-    if Vu is not None:
-        asm.ctx.call("fecx_update_field_unknowns", _ptr(Vu), _ptr(p.hvp_scratch_field))
+    bc = _ptr(p._bc_vals) if len(asm.dof.dirichlet_dofs) else None
+    asm.ctx.call("fecx_update_fields", bc, _ptr(Uu), _ptr(p.field), None if Vu is None else _ptr(Vu),
+                 None if Vu is None else _ptr(p.hvp_scratch_field))
 
 
 def _check_vec(asm, x, name, n=None):

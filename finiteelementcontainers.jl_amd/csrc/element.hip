@@ -860,7 +860,7 @@ __global__ __launch_bounds__(256) void element_kernel(ElementArgs args) {
       for (int idx = done + wl; idx < total; idx += 64) out[idx] = src[idx];
     }
   }
-  if (bad) atomicOr(args.flag, 1);
+  if (bad) raise_flag(args.flag);
 }
 
 template <int KIND, int NF, int PHYS, bool G64 = false>
@@ -1174,7 +1174,7 @@ void fused_hex8_kernel(ElementArgs args, FusedArgs f) {
       // no barrier here: element_eval's first barrier comes before its first write to the work area
     }
   }
-  if (bad) atomicOr(args.flag, 1);
+  if (bad) raise_flag(args.flag);
 }
 
 // The two scatter designs the fused kernel is measured against, on the same structured hex8 meshes and the same
@@ -1257,7 +1257,7 @@ void scatter_hex8_kernel(ElementArgs args, FusedArgs f, int colour) {
         }
     }
   }
-  if (bad) atomicOr(args.flag, 1);
+  if (bad) raise_flag(args.flag);
 }
 
 // scatter 1: FP64 atomics, 2: element colouring; vals and R zero-filled by the caller

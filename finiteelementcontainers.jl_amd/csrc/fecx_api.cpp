@@ -45,8 +45,6 @@ struct Prof {
   }
 };
 
-__global__ void zero_int_kernel(int* p) { *p = 0; }
-
 void check_device(fecx_ctx* ctx) {
   require(ctx->device >= 0, FECX_ERR_STATE, "host-only context (device -1) cannot run kernels");
 }
@@ -57,6 +55,15 @@ void check_ready(fecx_ctx* ctx) {
   require(ctx->has_dofs, FECX_ERR_STATE, "fecx_set_dofs has not been called");
   require(ctx->has_pattern, FECX_ERR_STATE, "fecx_build_pattern has not been called");
   require(ctx->has_material, FECX_ERR_STATE, "fecx_set_material has not been called");
+}
+
+fecx::DofMap dof_map(fecx_ctx* ctx) {
+  fecx::DofMap m{};
+  m.n = ctx->nn * ctx->nf;
+  m.mask = get<uint64_t>(ctx, "dof_mask");
+  m.base = get<int64_t>(ctx, "dof_base");
+  m.full = ctx->condensed ? 1 : 0;
+  return m;
 }
 
 fecx::ElementArgs element_args(fecx_ctx* ctx, const double* U, const double* V) {
@@ -73,7 +80,7 @@ fecx::ElementArgs element_args(fecx_ctx* ctx, const double* U, const double* V) 
   a.st_new = get<float>(ctx, "state_new");
   a.Rel = get<float>(ctx, "Rel");
   a.Kel = get<float>(ctx, "Kel");
-  a.flag = get<int>(ctx, "flag");
+  a.flag = ctx->flag_host;
   a.mp = ctx->mp;
   a.fp64_geometry = ctx->fp64_geometry ? 1 : 0;
   return a;
@@ -181,20 +188,21 @@ int scatter_path(fecx_ctx* ctx, int mode, bool surrogate, bool noalloc) {
   return FECX_SCATTER_TWO_PHASE;
 }
 
-// The numeric flag before a launch: cleared on the device only if the last read-back did not find it clear.
-int* arm_flag(fecx_ctx* ctx) {
-  int* flag = get<int>(ctx, "flag");
-  if (ctx->flag_dirty) zero_int_kernel<<<1, 1, 0, ctx->stream>>>(flag);
-  ctx->flag_dirty = true;  // until this call reads it back as clear
+// The numeric flag before a launch: cleared only if the last look did not find it clear (a call that raised it, or that
+// stopped before it looked and may have left kernels running).
+void arm_flag(fecx_ctx* ctx) {
   require(ctx->flag_host != nullptr, FECX_ERR_STATE, "no host flag word");
-  return flag;
+  if (ctx->flag_dirty) {
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    *(volatile int*)ctx->flag_host = 0;
+  }
+  ctx->flag_dirty = true;  // until this call finds it clear
 }
 
-// Reads the flag back (pinned word, stream-ordered after the kernels) and waits for the stream.
-int read_flag(fecx_ctx* ctx, const int* flag) {
-  HIPCHK(hipMemcpyAsync(ctx->flag_host, flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+// Waits for the stream and looks at the flag.
+int read_flag(fecx_ctx* ctx) {
   HIPCHK(hipStreamSynchronize(ctx->stream));
-  const int h = *ctx->flag_host;
+  const int h = *(volatile int*)ctx->flag_host;
   ctx->flag_dirty = h != 0;
   return h;
 }
@@ -232,7 +240,7 @@ void assemble(fecx_ctx* ctx, int mode, const double* U, const double* V, double*
   }
   Prof prof(ctx);
   if (noalloc) prof.ctx = nullptr;  // no HIP events
-  int* flag = arm_flag(ctx);
+  arm_flag(ctx);
   fecx::ElementArgs ea = element_args(ctx, U, V);
   ea.Kel = kel;
   ea.Rel = rel;
@@ -273,7 +281,7 @@ void assemble(fecx_ctx* ctx, int mode, const double* U, const double* V, double*
     }
     require(rc == 0, FECX_ERR_UNSUPPORTED, "no kernel of this scatter design for this nf / physics");
     HIPCHK(hipGetLastError());
-    const int hflag = read_flag(ctx, flag);
+    const int hflag = read_flag(ctx);
     prof.finish();
     require(hflag == 0, FECX_ERR_NUMERIC, "element kernel met a non-positive Jacobian determinant or a NaN");
     return;
@@ -326,7 +334,7 @@ void assemble(fecx_ctx* ctx, int mode, const double* U, const double* V, double*
     require(rc == 0, FECX_ERR_UNSUPPORTED, "no reduction kernel for this element kind / nf");
     HIPCHK(hipGetLastError());
   }
-  const int hflag = read_flag(ctx, flag);
+  const int hflag = read_flag(ctx);
   prof.finish();
   if (surrogate) fecx::surrogate_qp_finish(ctx);
   require(hflag == 0, FECX_ERR_NUMERIC, "element kernel met a non-positive Jacobian determinant or a NaN");
@@ -340,7 +348,7 @@ void assemble_mass(fecx_ctx* ctx, int what, double density, const double* V, dou
           "mesh, dofs and pattern must be set before a mass assembly");
   require(std::isfinite(density), FECX_ERR_ARG, "density must be finite");
   Prof prof(ctx);
-  int* flag = arm_flag(ctx);
+  arm_flag(ctx);
   fecx::ElementArgs ea = element_args(ctx, nullptr, V);
   int rc = 0;
   prof.run("mass_element", ctx->stream, [&] { rc = fecx::launch_mass(ctx->kind, ctx->nf, what, ea, (float)density, ctx->stream); });
@@ -356,7 +364,7 @@ void assemble_mass(fecx_ctx* ctx, int what, double density, const double* V, dou
   });
   require(rc == 0, FECX_ERR_UNSUPPORTED, "no reduction kernel for this element kind / nf");
   HIPCHK(hipGetLastError());
-  const int hflag = read_flag(ctx, flag);
+  const int hflag = read_flag(ctx);
   prof.finish();
   require(hflag == 0, FECX_ERR_NUMERIC, "mass kernel met a non-positive Jacobian determinant");
 }
@@ -376,9 +384,9 @@ int fecx_create(fecx_ctx** out, int device) {
   fecx_ctx* ctx = new fecx_ctx();
   ctx->device = device;
   int rc = guard(ctx, [&] {
-    (void)dev(ctx, "flag", sizeof(int));
     if (device >= 0) {
       HIPCHK(hipHostMalloc((void**)&ctx->flag_host, sizeof(int), hipHostMallocDefault));
+      *ctx->flag_host = 0;
       HIPCHK(hipHostMalloc((void**)&ctx->cg_done_host, sizeof(int), hipHostMallocDefault));
       // the allocation-free entry point's per-device scratch address, looked up once per device, device current
       require(fecx::noalloc_setup(device) == FECX_OK, FECX_ERR_HIP, "scratch symbol lookup failed");
@@ -482,7 +490,13 @@ int fecx_set_dofs(fecx_ctx* ctx, int nf, const int64_t* dirichlet, int64_t ndir)
     std::vector<int64_t> u0(ctx->unknown_dofs.size()), d0(ndir);
     for (size_t i = 0; i < u0.size(); ++i) u0[i] = ctx->unknown_dofs[i] - 1;
     for (int64_t i = 0; i < ndir; ++i) d0[i] = dirichlet[i] - 1;
-    upload(ctx, "unknown_idx", u0);
+    // the unknown dofs as bits, 64 to a word, and the number of unknowns before each word
+    std::vector<uint64_t> mask((size_t)((N + 63) / 64), 0);
+    std::vector<int64_t> base(mask.size(), 0);
+    for (int64_t d : u0) mask[(size_t)(d >> 6)] |= uint64_t(1) << (d & 63);
+    for (size_t w = 1; w < mask.size(); ++w) base[w] = base[w - 1] + __builtin_popcountll(mask[w - 1]);
+    upload(ctx, "dof_mask", mask);
+    upload(ctx, "dof_base", base);
     upload(ctx, "dirichlet_idx", d0);
     ctx->has_dofs = true;
     ctx->has_pattern = false;
@@ -901,23 +915,26 @@ int fecx_assemble_mass_action(fecx_ctx* ctx, double density, const double* V, do
   });
 }
 
-int fecx_update_field_unknowns(fecx_ctx* ctx, const double* Uu, double* U) {
+int fecx_update_fields(fecx_ctx* ctx, const double* bc, const double* Uu, double* U, const double* Vu, double* V) {
   return guard(ctx, [&] {
     check_device(ctx);
     require(ctx->has_dofs, FECX_ERR_STATE, "fecx_set_dofs has not been called");
-    const int64_t n = (int64_t)ctx->unknown_dofs.size();
-    if (ctx->condensed) fecx::launch_copy_indexed(n, get<int64_t>(ctx, "unknown_idx"), Uu, U, ctx->stream);
-    else fecx::launch_scatter_unknowns(n, get<int64_t>(ctx, "unknown_idx"), Uu, U, ctx->stream);
+    const fecx::DofMap m = dof_map(ctx);
+    fecx::launch_update_fields(m, ctx->dirichlet.empty() ? nullptr : bc, Uu, U, Vu, V, ctx->stream);
     HIPCHK(hipGetLastError());
   });
+}
+
+int fecx_update_field_unknowns(fecx_ctx* ctx, const double* Uu, double* U) {
+  return fecx_update_fields(ctx, nullptr, Uu, U, nullptr, nullptr);
 }
 
 int fecx_update_field_dirichlet(fecx_ctx* ctx, const double* vals, double* U) {
   return guard(ctx, [&] {
     check_device(ctx);
     require(ctx->has_dofs, FECX_ERR_STATE, "fecx_set_dofs has not been called");
-    fecx::launch_scatter_unknowns((int64_t)ctx->dirichlet.size(), get<int64_t>(ctx, "dirichlet_idx"), vals, U,
-                                  ctx->stream);
+    fecx::launch_scatter_indexed((int64_t)ctx->dirichlet.size(), get<int64_t>(ctx, "dirichlet_idx"), vals, U,
+                                 ctx->stream);
     HIPCHK(hipGetLastError());
   });
 }
@@ -926,8 +943,7 @@ int fecx_extract_field_unknowns(fecx_ctx* ctx, const double* U, double* Uu) {
   return guard(ctx, [&] {
     check_device(ctx);
     require(ctx->has_dofs, FECX_ERR_STATE, "fecx_set_dofs has not been called");
-    fecx::launch_gather_unknowns((int64_t)ctx->unknown_dofs.size(), get<int64_t>(ctx, "unknown_idx"), U, Uu,
-                                 ctx->stream);
+    fecx::launch_extract_unknowns(dof_map(ctx), U, Uu, ctx->stream);
     HIPCHK(hipGetLastError());
   });
 }

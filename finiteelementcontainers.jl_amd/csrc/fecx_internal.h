@@ -147,7 +147,7 @@ struct ElementArgs {
   float* st_new;
   float* Rel;               // ne x ndof   (residual or action output)
   float* Kel;               // ne x npairs x nf*nf
-  int* flag;                // error flag (bit 1: bad Jacobian / NaN)
+  int* flag;                // error flag, a pinned host word (bad Jacobian / NaN)
   float* hq;                // MODE_QPGRAD output: ne x nq x (nf*nd) gradients, element storage order
   const float* qpmat;       // surrogate materials: ne x nq x (nf*nd + NC) stress and tangent data
   MatParams mp;
@@ -211,11 +211,21 @@ constexpr int NOALLOC_MAX_DEVICES = 64;
 int noalloc_setup(int device);
 void* noalloc_scratch(int device);
 
-// DOF plumbing
-void launch_scatter_unknowns(int64_t n, const int64_t* idx, const double* src, double* dst, hipStream_t s);
-void launch_gather_unknowns(int64_t n, const int64_t* idx, const double* src, double* dst, hipStream_t s);
-// dst[idx[i]] = src[idx[i]] (condensed mode: full-length unknown vectors)
-void launch_copy_indexed(int64_t n, const int64_t* idx, const double* src, double* dst, hipStream_t s);
+// DOF plumbing: the unknown dofs of a field as a bit mask, with the number of unknowns before each 64-bit word. A dof's
+// place in the unknown vector follows from them (12 bytes per 64 dofs), and a fixed dof's place in the Dirichlet list,
+// which is sorted too.
+struct DofMap {
+  int64_t n;             // dofs of the full field
+  const uint64_t* mask;
+  const int64_t* base;
+  int full;              // condensed mode: the unknown vectors are full length
+};
+// U = Uu at the unknown dofs and bc at the fixed ones (bc null: they stay); V = Vu at the unknown dofs, if given
+void launch_update_fields(const DofMap& m, const double* bc, const double* Uu, double* U, const double* Vu, double* V,
+                          hipStream_t s);
+void launch_extract_unknowns(const DofMap& m, const double* U, double* Uu, hipStream_t s);
+// dst[idx[i]] = src[i]
+void launch_scatter_indexed(int64_t n, const int64_t* idx, const double* src, double* dst, hipStream_t s);
 
 }  // namespace fecx
 
@@ -289,10 +299,10 @@ struct fecx_ctx {
   bool fp64_geometry = false;  // tet10 element geometry, field gradient and stress in FP64 (fecx_set_fp64_geometry)
   hipStream_t stream2 = nullptr;
   std::vector<hipEvent_t> events;
-  // numeric error flag: device word set by the kernels, read back through a pinned host word after every assembly;
-  // cleared on the device only when the last read-back did not find it clear (an error, or a call that stopped early)
+  // numeric error flag: a pinned host word that the kernels set (raise_flag), looked at after every assembly and cleared
+  // only when the last look did not find it clear (an error, or a call that stopped early)
   int* flag_host = nullptr;
-  bool flag_dirty = true;
+  bool flag_dirty = false;
   // conjugate gradients: pinned convergence word and the events that mark the enqueued batches of iterations
   int* cg_done_host = nullptr;
   std::vector<hipEvent_t> cg_events;

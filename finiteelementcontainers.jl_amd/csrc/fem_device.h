@@ -518,6 +518,12 @@ struct Mat<FECX_NH_SURROGATE> : Mat<FECX_NEOHOOKEAN> {
   static constexpr bool FROM_QP = true;
 };
 
+// The numeric flag: a pinned host word that a kernel sets where it meets a bad element, and the call looks at once its
+// stream is done (no copy, no device word to clear). Any number of lanes store the same value.
+__device__ __forceinline__ void raise_flag(int* flag) {
+  __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ------------------------------------------------------------------ LDS staging shared by the element and mass kernels
 typedef float f32x4 __attribute__((ext_vector_type(4)));  // 16-byte moves (nontemporal stores need a vector type)
 

@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256) void mass_kernel(ElementArgs args, float rho) 
       for (int idx = done + wl; idx < total; idx += 64) out[idx] = src[idx];
     }
   }
-  if (bad) atomicOr(args.flag, 1);
+  if (bad) raise_flag(args.flag);
 }
 
 template <int KIND, int NF>

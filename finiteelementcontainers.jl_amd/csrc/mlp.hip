@@ -504,7 +504,7 @@ __global__ __launch_bounds__(256) void material_kernel(MatBatchArgs a) {
     }
   }
   if (!valid || h != 0) return;
-  if (bad && a.flag) atomicOr(a.flag, 1);
+  if (bad && a.flag) raise_flag(a.flag);
   if (a.hq) {
     float* q = a.qpmat + i * (9 + NC);
 #pragma unroll

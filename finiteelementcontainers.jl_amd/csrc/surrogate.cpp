@@ -144,7 +144,7 @@ void surrogate_qp_pass(fecx_ctx* ctx, const float* hq, float* qpmat, hipStream_t
   a.st_old = get<float>(ctx, "state_old");
   a.st_new = get<float>(ctx, "state_new");
   a.qpmat = qpmat;
-  a.flag = get<int>(ctx, "flag");
+  a.flag = ctx->flag_host;
   a.mp.phys = ctx->mp.phys == FECX_J2_SURROGATE ? FECX_J2 : FECX_NEOHOOKEAN;
   a.accept = (uint8_t*)fecx_api::get<uint8_t>(ctx, "sg_accept");
   if (!a.accept || fecx_api::get_bytes(ctx, "sg_accept") < (size_t)a.n) {
@@ -410,12 +410,11 @@ int fecx_qp_gradients(fecx_ctx* ctx, const double* U, float* Hq) {
     ea.xhi = get<float>(ctx, "xhi");
     ea.xlo = get<float>(ctx, "xlo");
     ea.U = U;
-    ea.flag = get<int>(ctx, "flag");
+    ea.flag = ctx->flag_host;  // not looked at here: the next assembly clears it first
+    ctx->flag_dirty = true;
     ea.mp = ctx->mp;
     ea.fp64_geometry = ctx->fp64_geometry ? 1 : 0;
     ea.hq = (float*)dev_atleast(ctx, "hq", sizeof(float) * nqp * 9);
-    HIPCHK(hipMemsetAsync(ea.flag, 0, sizeof(int), ctx->stream));
-    ctx->flag_dirty = true;  // not read back here: the next assembly clears it first
     require(fecx::launch_element(ctx->kind, ctx->nf, fecx::MODE_QPGRAD, ea, ctx->stream) == 0, FECX_ERR_UNSUPPORTED,
             "no gradient kernel for this element kind");
     // storage order -> element order: row e of Hq is row epos[e] of the storage-ordered buffer

@@ -244,6 +244,10 @@ int fecx_update_field_unknowns(fecx_ctx* ctx, const double* Uu, double* U);
  * update_field_dirichlet_bcs! (src/bcs/DirichletBCs.jl:411-418). */
 int fecx_update_field_dirichlet(fecx_ctx* ctx, const double* vals, double* U);
 
+/* _update_for_assembly! (src/Parameters.jl:404-442) in one launch: U[dirichlet_dofs] = bc (unless bc is NULL),
+ * U[unknown_dofs] = Uu, and, for the actions, V[unknown_dofs] = Vu (Vu and V may be NULL). */
+int fecx_update_fields(fecx_ctx* ctx, const double* bc, const double* Uu, double* U, const double* Vu, double* V);
+
 /* Uu = U[unknown_dofs]: extract_field_unknowns! (src/DofManagers.jl:203-213). */
 int fecx_extract_field_unknowns(fecx_ctx* ctx, const double* U, double* Uu);
 
