@@ -10,12 +10,12 @@
 // src/assemblers/Assemblers.jl:72-87 restated as an owner-computes gather).
 // These kernels share this contract (launch_buckets routes the light rows, then the heavy ones):
 //   reduce_scalar_hex8_kernel   scalar hex8 light rows: lanes add their words into LDS slot accumulators;
-//   reduce_scatter_kernel       3-field light rows of up to 32 blocks, and the tet10 heavy rows (scalar and 3-field)
-//                               of up to 72 blocks: the same scatter, 32 or 64 lanes per row;
+//   reduce_scatter_kernel       light rows of up to 32 blocks of 2 and 3 fields and of scalar tet10, and the tet10 heavy rows
+//                               (scalar and 3-field) of up to 72 blocks: the same scatter, 16, 32 or 64 lanes per row;
 //   reduce_merged_kernel        3-field tet10 meshes whose rows have at most 65 blocks: both buckets of
 //                               reduce_scatter_kernel in one launch, their work-groups interleaved along the Morton curve;
-//   reduce_rows_kernel          slot-owner lanes for everything else: light scalar tet10/quad4 rows, 3-field light
-//                               rows of more than 32 blocks, heavy hex8/quad4 rows and tet10 rows of more than 72;
+//   reduce_rows_kernel          slot-owner lanes for everything else: light scalar quad4 rows, heavy hex8/quad4 rows and
+//                               tet10 rows of more than 72 blocks;
 //   reduce_expand_kernel        mass matrices of 2 or 3 fields, from one word per node pair (blocks m I);
 //   reduce_vector_kernel / reduce_vector_group_kernel   calls without CSR values (one thread, or 16 lanes, per row).
 // All sum a slot's (or a row's) contributions in ascending incidence order, so every form gives the same bits.
@@ -128,22 +128,11 @@ void reduce_rows_kernel(ReduceArgs a) {
   for (int pass = 0; pass < maxpass; ++pass) {
     const int base = pass * CHK;
     const int cnt = min(CHK, ninc - base);  // may be <= 0 for this node
-    // padded light rows (scalar kernels only): the 8 slots at 8 pos are loaded without waiting for the row descriptor
-    // (unused slots hold a valid incidence and are never summed: every later loop stops at cnt). The vector-row
-    // kernels keep the plain form, which holds their register count below the next occupancy step.
-    bool stage;
-    int64_t c;
-    if constexpr (NF == 1) {
-      stage = (CHK == CH && a.padded) ? (valid && lane < CH) : (lane < cnt);
-      c = (CHK == CH && a.padded) ? pos * CH + lane : (int64_t)c0 + base + lane;
-    } else {
-      stage = lane < cnt;
-      c = c0 + base + lane;
-    }
-    if (stage) {
+    const int64_t c = (int64_t)c0 + base + lane;
+    if (lane < cnt) {
       const int32_t v = a.vent[c];
       s_v[grp][lane] = v;
-      const uint32_t* sl = reinterpret_cast<const uint32_t*>(a.vslot) + (int64_t)c * VW;
+      const uint32_t* sl = reinterpret_cast<const uint32_t*>(a.vslot) + c * VW;
 #pragma unroll
       for (int q = 0; q < VW; ++q) s_w[grp][lane][q] = sl[q];
       if (a.R) {
@@ -593,7 +582,7 @@ static int launch_lpr(const ReduceArgs& a, int maxdeg, hipStream_t s) {
   const int sw = maxdeg <= lpr ? 1 : (maxdeg <= 2 * lpr ? 2 : 4);
   // more than one sweep on the narrow scalar rows, where wider rows move to the next lane count first, and on the
   // 128-lane rows (129..256 blocks: vertex rows of unstructured tet10 meshes); wider rows are refused
-  if (maxdeg > sw * lpr || (sw == 4 && lpr != 8) || (sw > 1 && lpr > 16 && lpr != 128)) return -1;
+  if (maxdeg > sw * lpr || (sw == 4 && lpr != 8) || (sw > 1 && lpr != 8 && lpr != 128)) return -1;
   const int64_t npw = RED_THREADS / lpr;
   int64_t grid = (a.p1 - a.p0 + npw - 1) / npw;
   grid = (grid + 7) / 8 * 8;  // XCD remap needs a multiple of 8
@@ -606,9 +595,7 @@ static int launch_lpr(const ReduceArgs& a, int maxdeg, hipStream_t s) {
       return 0;
     }
   }
-  if (lpr == 16 && sw == 1) reduce_rows_kernel<NF, NNPE, 16, 1><<<g, RED_THREADS, 0, s>>>(a);
-  else if (lpr == 16) reduce_rows_kernel<NF, NNPE, 16, 2><<<g, RED_THREADS, 0, s>>>(a);
-  else if (lpr == 32) reduce_rows_kernel<NF, NNPE, 32, 1><<<g, RED_THREADS, 0, s>>>(a);
+  if (lpr == 32) reduce_rows_kernel<NF, NNPE, 32, 1><<<g, RED_THREADS, 0, s>>>(a);
   else if (lpr == 64) reduce_rows_kernel<NF, NNPE, 64, 1><<<g, RED_THREADS, 0, s>>>(a);
   else if (sw == 1) reduce_rows_kernel<NF, NNPE, 128, 1, RED_HEAVY_CH><<<g, RED_THREADS, 0, s>>>(a);
   else reduce_rows_kernel<NF, NNPE, 128, 2, RED_HEAVY_CH><<<g, RED_THREADS, 0, s>>>(a);
@@ -623,10 +610,9 @@ static int launch_buckets(const ReduceArgs& a, hipStream_t s) {
   ReduceArgs lo = a, hi = a;
   lo.p1 = std::min(a.p1, std::max(a.p0, a.nlight));
   hi.p0 = std::max(a.p0, a.nlight);
-  // Light rows take one pass, so their launch can skip the pass-count vote and its barriers: measured -2.6 % (Poisson
-  // hex8 128^3) and -0.8 % (neo-Hookean hex8 96^3), but +3.4 % on the tet10 edge rows, which keep the vote.
+  // light rows take one pass, so their launch can skip the slot-owner kernel's pass-count vote and its barriers
   static_assert(CH >= 8, "light rows have at most 8 incidences and must take one pass");
-  lo.onepass = NNPE == 8 ? 1 : 0;
+  lo.onepass = 1;
   hi.onepass = 0;
   // direct slot addressing measured -1 % (scalar rows) and +0.8 % (vector rows) on the matrix reduction
   lo.padded = (NF == 1 && a.npad >= lo.p1) ? 1 : 0;
@@ -638,8 +624,6 @@ static int launch_buckets(const ReduceArgs& a, hipStream_t s) {
       int64_t grid = (lo.p1 - lo.p0 + RED_THREADS / 8 - 1) / (RED_THREADS / 8);
       grid = (grid + 7) / 8 * 8;  // XCD remap needs a multiple of 8
       reduce_scalar_hex8_kernel<32><<<(unsigned)grid, RED_THREADS, 0, s>>>(lo);
-    } else {
-      rc = launch_lpr<NF, NNPE>(lo, a.maxdeg_light, s);
     }
   } else if constexpr (NF == 3) {
     if (NNPE == 10 && a.merged && a.nmerged > 0 && a.p0 == 0 && a.nlight < a.p1 && a.maxdeg_light <= 32 &&
@@ -649,16 +633,25 @@ static int launch_buckets(const ReduceArgs& a, hipStream_t s) {
       else reduce_merged_kernel<false><<<(unsigned)grid, RED_THREADS, 0, s>>>(a);
       return 0;
     }
-    if (lo.p1 > lo.p0 && a.maxdeg_light <= 32) {
+    if (lo.p1 > lo.p0) {
+      if (a.maxdeg_light > 32) return -1;
       int64_t grid = (lo.p1 - lo.p0 + RED_THREADS / 32 - 1) / (RED_THREADS / 32);
       grid = (grid + 7) / 8 * 8;  // XCD remap needs a multiple of 8
       if (a.rmap) reduce_scatter_kernel<true, NF, NNPE, 32, CH, 32><<<(unsigned)grid, RED_THREADS, 0, s>>>(lo);
       else reduce_scatter_kernel<false, NF, NNPE, 32, CH, 32><<<(unsigned)grid, RED_THREADS, 0, s>>>(lo);
-    } else {
-      rc = launch_lpr<NF, NNPE>(lo, a.maxdeg_light, s);
     }
-  } else {
+  } else if constexpr (NF == 1 && NNPE == 4) {
+    // two to four words per lane would leave half the lanes idle: the slot-owner kernel is as fast (64^2: 29.6 against 29.4 us
+    // a step, 400 x 300: 41.5 against 42.9)
     rc = launch_lpr<NF, NNPE>(lo, a.maxdeg_light, s);
+  } else if (lo.p1 > lo.p0) {
+    // scalar tet10 and plane strain, 16 lanes per row: steps on Poisson tet10 28^3 x 6 132 -> 109 us, 8 x 9 x 7 x 6 45 -> 36 us,
+    // plane-strain quad4 400 x 450 95 -> 69 us against the slot-owner kernel
+    if (a.maxdeg_light > 32) return -1;
+    constexpr int LPR = 16;
+    const int64_t grid = ((lo.p1 - lo.p0 + RED_THREADS / LPR - 1) / (RED_THREADS / LPR) + 7) / 8 * 8;  // multiple of 8
+    if (NF > 1 && a.rmap) reduce_scatter_kernel<NF != 1, NF, NNPE, LPR, CH, 32><<<(unsigned)grid, RED_THREADS, 0, s>>>(lo);
+    else reduce_scatter_kernel<false, NF, NNPE, LPR, CH, 32><<<(unsigned)grid, RED_THREADS, 0, s>>>(lo);
   }
   if (rc != 0 || hi.p1 <= hi.p0) return rc;
   if constexpr (NNPE == 10) {
