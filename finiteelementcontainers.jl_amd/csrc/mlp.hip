@@ -339,11 +339,11 @@ __device__ __forceinline__ bool j2_surrogate(const MatParams& mp, const float* H
 #pragma unroll
   for (int i = 0; i < 9; ++i) ee[i] = eps[i] - epo[i] - dep[i];
   const float tre = ee[0] + ee[4] + ee[8];
-  float r = 0.0f;
+  float r = 0.0f;  // the largest deviation, divided once (division by a positive number keeps the order, rounding included)
 #pragma unroll
   for (int i = 0; i < 9; ++i) {
     const float se = 2 * mu * ee[i] + ((i % 4 == 0) ? (kap - 2 * mu / 3) * tre : 0.0f);
-    r = fmaxf(r, fabsf(sig[i] - se) / sy);
+    r = fmaxf(r, fabsf(sig[i] - se));
   }
   // yield
   const float trs = (sig[0] + sig[4] + sig[8]) / 3;
@@ -353,12 +353,13 @@ __device__ __forceinline__ bool j2_surrogate(const MatParams& mp, const float* H
   const float snorm = sqrtf(sn2);
   const float f = snorm - r23 * (sy + Hh * (so[6] + dal));
   const bool plastic = dal > tol * eref;
-  r = fmaxf(r, plastic ? fabsf(f) / sy : fmaxf(f, 0.0f) / sy);
+  r = fmaxf(0.0f, fmaxf(r, plastic ? fabsf(f) : fmaxf(f, 0.0f)) / sy);
   // flow rule
   const float inv = snorm > 0.0f ? 1.0f / snorm : 0.0f;
+  float rf = fmaxf(-dal, 0.0f);
 #pragma unroll
-  for (int i = 0; i < 9; ++i) r = fmaxf(r, fabsf(dep[i] - r32 * fmaxf(dal, 0.0f) * s[i] * inv) / eref);
-  r = fmaxf(r, fmaxf(-dal, 0.0f) / eref);
+  for (int i = 0; i < 9; ++i) rf = fmaxf(rf, fabsf(dep[i] - r32 * fmaxf(dal, 0.0f) * s[i] * inv));
+  r = fmaxf(r, rf / eref);
   if (!(r <= tol)) return false;
 #pragma unroll
   for (int i = 0; i < 9; ++i) P[i] = sig[i];
@@ -416,11 +417,13 @@ __device__ __forceinline__ bool nh_surrogate(const MatParams& mp, const float* H
 #pragma unroll
     for (int j = 0; j < 3; ++j) FiT[i * 3 + j] = F[i * 3 + 0] * Ci[0 * 3 + j] + F[i * 3 + 1] * Ci[1 * 3 + j] + F[i * 3 + 2] * Ci[2 * 3 + j];
   const float ps = (mu + lam) * hmax;
+  float rp = 0.0f;
 #pragma unroll
   for (int i = 0; i < 9; ++i) {
     const float pp = mu * (F[i] - FiT[i]) + lam * lnJ * FiT[i];
-    r = fmaxf(r, fabsf(y[i] - pp) / ps);
+    rp = fmaxf(rp, fabsf(y[i] - pp));
   }
+  r = fmaxf(r, rp / ps);
   if (!(r <= tol)) return false;
 #pragma unroll
   for (int i = 0; i < 9; ++i) { P[i] = y[i]; C[i] = FiT[i]; }
@@ -429,7 +432,12 @@ __device__ __forceinline__ bool nh_surrogate(const MatParams& mp, const float* H
 }
 
 // ------------------------------------------------------------------ batched material update
-// One wavefront per 32 samples (both lane halves carry the same sample; half 0 stores). Sources and sinks:
+// One wavefront per 64 samples, lane = sample: features, residual check, decode and stores are done once per sample, and the
+// network runs two 32-sample tiles at a time (mlp_forward_wave). Bound by VALU: a hidden activation costs five VALU operations,
+// two transcendental ones (quarter rate) and half a conversion, so 2,097,152 J2 samples with 384 each need about 0.4 ms, and
+// their 245 MB in and out 0.06 ms. With one 32-sample tile per wavefront, both lane halves doing the same check and every weight
+// operand loaded per tile: J2 2,097,152 samples 888 us, now 457; neo-Hookean 2,000,000 873 -> 533, 70,000 85 -> 72; J2 5,000
+// 46 -> 41. Sources and sinks:
 //   batch mode    : in (n x IN_W raw) -> out (n x OUT_W raw)
 //   assembly mode : hq (n x 9 quadrature-point gradients, n = ne x nq in element storage order) and the element's
 //                   state (via eperm) -> qpmat (n x (9 + NC): P, compact tangent) and state_new
@@ -439,10 +447,10 @@ __global__ __launch_bounds__(256) void material_kernel(MatBatchArgs a) {
   using FT = Feat<ARCH>;
   constexpr bool J2 = ARCH == FECX_MLP_J2;
   constexpr int NC = J2 ? Mat<FECX_J2>::NC : Mat<FECX_NEOHOOKEAN>::NC;
-  const int lane = threadIdx.x % 64, h = lane >> 5;
+  const int lane = threadIdx.x % 64;
   const int64_t tile = (int64_t)blockIdx.x * 4 + threadIdx.x / 64;
-  const int64_t i = tile * 32 + lane % 32;
-  if (tile * 32 >= a.n) return;  // wave-uniform
+  const int64_t i = tile * 64 + lane;
+  if (tile * 64 >= a.n) return;  // wave-uniform
   const bool valid = i < a.n;
   float H[9] = {}, so[7] = {};
   int64_t sidx = 0;
@@ -473,7 +481,7 @@ __global__ __launch_bounds__(256) void material_kernel(MatBatchArgs a) {
 #pragma unroll
     for (int c = 0; c < 7; ++c) raw[9 + c] = so[c];
     normalized_features<ARCH>(a.m, raw, x);
-    float yn[32];
+    float yn[16];
     mlp_forward_wave<A>(a.m, x, yn, lane);
 #pragma unroll
     for (int o = 0; o < FT::OUT_W; ++o) y[o] = yn[o] * a.m.out_scale[o] + a.m.out_shift[o];
@@ -487,9 +495,9 @@ __global__ __launch_bounds__(256) void material_kernel(MatBatchArgs a) {
         if constexpr (J2) ok = j2_surrogate(a.mp, H, so, y, tol, P, sn, C);
         else ok = nh_surrogate(a.mp, H, y, tol, P, C);
       }
-      if (a.accept && !frozen && h == 0) a.accept[i] = ok ? 1 : 0;
+      if (a.accept && !frozen) a.accept[i] = ok ? 1 : 0;
     }
-    const uint64_t fb = __ballot(valid && h == 0 && !ok);
+    const uint64_t fb = __ballot(valid && !ok);
     if (lane == 0 && fb && a.nfallback) atomicAdd(a.nfallback, (unsigned long long)__popcll(fb));
   }
   if (valid && !ok) {  // the plain model: the fallback, or the whole update when SURR is off
@@ -503,7 +511,7 @@ __global__ __launch_bounds__(256) void material_kernel(MatBatchArgs a) {
       for (int c = 0; c < 7; ++c) y[6 + c] = sn[c] - so[c];
     }
   }
-  if (!valid || h != 0) return;
+  if (!valid) return;
   if (bad && a.flag) raise_flag(a.flag);
   if (a.hq) {
     float* q = a.qpmat + i * (9 + NC);
@@ -526,17 +534,17 @@ template <int ARCH>
 __global__ __launch_bounds__(256) void mlp_forward_kernel(MatBatchArgs a) {
   using A = Arch<ARCH>;
   using FT = Feat<ARCH>;
-  const int lane = threadIdx.x % 64, h = lane >> 5;
-  const int64_t tile = (int64_t)blockIdx.x * 4 + threadIdx.x / 64;
-  const int64_t i = tile * 32 + lane % 32;
-  if (tile * 32 >= a.n) return;
+  const int lane = threadIdx.x % 64;
+  const int64_t tile = (int64_t)blockIdx.x * 4 + threadIdx.x / 64;  // 64 samples per wavefront
+  const int64_t i = tile * 64 + lane;
+  if (tile * 64 >= a.n) return;
   const bool valid = i < a.n;
-  float raw[16] = {}, x[16], yn[32];
+  float raw[16] = {}, x[16], yn[16];
 #pragma unroll
   for (int c = 0; c < FT::IN_W; ++c) raw[c] = valid ? a.in[i * FT::IN_W + c] : 0.0f;
   normalized_features<ARCH>(a.m, raw, x);
   mlp_forward_wave<A>(a.m, x, yn, lane);
-  if (valid && h == 0) {
+  if (valid) {
 #pragma unroll
     for (int o = 0; o < FT::OUT_W; ++o) a.out[i * FT::OUT_W + o] = yn[o] * a.m.out_scale[o] + a.m.out_shift[o];
   }
@@ -657,13 +665,13 @@ void mlp_launch_gather(int64_t n, int w, const int32_t* idx, const float* src, f
   if (n > 0) gather_rows_kernel<<<(unsigned)((n * w + 255) / 256), 256, 0, s>>>(n, w, idx, src, dst);
 }
 void mlp_launch_forward(int arch, const MatBatchArgs& a, hipStream_t s) {
-  const unsigned g = (unsigned)((a.n + 127) / 128);
+  const unsigned g = (unsigned)((a.n + 255) / 256);
   if (a.n == 0) return;
   if (arch == FECX_MLP_J2) mlp_forward_kernel<FECX_MLP_J2><<<g, 256, 0, s>>>(a);
   else mlp_forward_kernel<FECX_MLP_NH><<<g, 256, 0, s>>>(a);
 }
 void mlp_launch_material(int arch, bool surrogate, const MatBatchArgs& a, hipStream_t s) {
-  const unsigned g = (unsigned)((a.n + 127) / 128);
+  const unsigned g = (unsigned)((a.n + 255) / 256);
   if (a.n == 0) return;
   if (arch == FECX_MLP_J2) {
     if (surrogate) material_kernel<FECX_MLP_J2, true><<<g, 256, 0, s>>>(a);

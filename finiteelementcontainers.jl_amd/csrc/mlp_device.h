@@ -1,7 +1,7 @@
 // MLP building blocks on CDNA4 matrix cores (v_mfma_f32_32x32x16_bf16), shared by the surrogate training kernels
 // and the batched material kernels.
 //
-// Layout ("transposed" formulation): a wavefront evaluates 32 samples at once. A layer computes Z = W H + b with the
+// Layout ("transposed" formulation): an MFMA tile is 32 samples wide (training: one tile per wavefront; inference: two). A layer computes Z = W H + b with the
 // weights as the MFMA A operand (32 output features x 16 inputs per instruction) and the activations as the B operand
 // (16 inputs x 32 samples). Measured operand layouts on gfx950 (lane l, element i; h = l / 32):
 //   A[m = l % 32][k = 8 h + i],  B[k = 8 h + i][n = l % 32],  D register j: [m = 8 (j / 4) + 4 h + j % 4][n = l % 32].
@@ -163,74 +163,108 @@ __device__ __forceinline__ void pack_tiles(const f32x16* acc, bf16x8* hb) {
       for (int i = 0; i < 8; ++i) hb[2 * mt + s][i] = (__bf16)acc[mt][8 * s + i];
 }
 
-// GELU in place on the D tiles, then pack as B operands
-template <int OUT>
-__device__ __forceinline__ void gelu_pack(const f32x16* acc, bf16x8* hb) {
-#pragma unroll
-  for (int mt = 0; mt < OUT / 32; ++mt)
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int i = 0; i < 8; ++i) hb[2 * mt + s][i] = (__bf16)gelu(acc[mt][8 * s + i]);
-}
-
-// Z = W_l H + b for one hidden layer, with the bias, GELU and BF16 packing applied one 32-feature D tile at a time
-// straight into the next layer's B operands: one tile (16 registers) is live instead of P[l+1] / 2, so the inference
-// kernels fit more wavefronts per SIMD and one wavefront's activations overlap another's MFMAs. Same arithmetic, in the
-// same order, as mlp_layer followed by gelu_pack.
-template <class A, int L>
-__device__ __forceinline__ void mlp_layer_gelu(const MlpDev& m, const bf16x8* hb, bf16x8* hn, int lane) {
+// Z = W_l H + b for one hidden layer and T tiles of 32 samples, with the bias, GELU and BF16 packing applied one 32-feature D
+// tile at a time straight into the next layer's B operands: T D tiles (16 registers each) are live instead of P[l+1] / 2
+// registers per tile of samples. Every weight operand is loaded once for the T tiles: the weights of a wavefront come from L2
+// (76 KB for the J2 network, 144 KB for the neo-Hookean one, against 32 KB of L1). Same arithmetic, in the same order, as
+// mlp_layer followed by gelu.
+template <class A, int L, int T>
+__device__ __forceinline__ void mlp_layer_gelu(const MlpDev& m, const bf16x8 (&hb)[T][A::P[L] / 16],
+                                               bf16x8 (&hn)[T][A::P[L + 1] / 16], int lane) {
   constexpr int IN = A::P[L], OUT = A::P[L + 1];
   const bf16x8* w = m.wf + Offs<A>::wf(L);
   const float* b = m.bias + Offs<A>::bias(L);
   const int h = lane >> 5;
 #pragma unroll
   for (int mt = 0; mt < OUT / 32; ++mt) {
-    f32x16 c;
+    f32x16 c[T];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) c[j] = b[dreg_feature(mt, h, j)];
+    for (int j = 0; j < 16; ++j) {
+      const float bj = b[dreg_feature(mt, h, j)];
 #pragma unroll
-    for (int kb = 0; kb < IN / 16; ++kb)
-      c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[(mt * (IN / 16) + kb) * 64 + lane], hb[kb], c, 0, 0, 0);
+      for (int t = 0; t < T; ++t) c[t][j] = bj;
+    }
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
+    for (int kb = 0; kb < IN / 16; ++kb) {
+      const bf16x8 wv = w[(mt * (IN / 16) + kb) * 64 + lane];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) hn[2 * mt + s][i] = (__bf16)gelu(c[8 * s + i]);
+      for (int t = 0; t < T; ++t) c[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv, hb[t][kb], c[t], 0, 0, 0);
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) hn[t][2 * mt + s][i] = (__bf16)gelu(c[t][8 * s + i]);
+  }
+}
+// the output layer of T tiles (one D tile each)
+template <class A, int T>
+__device__ __forceinline__ void mlp_layer_out(const MlpDev& m, const bf16x8 (&hb)[T][A::P[A::NL - 1] / 16], f32x16 (&out)[T],
+                                              int lane) {
+  constexpr int L = A::NL - 1, IN = A::P[L];
+  const bf16x8* w = m.wf + Offs<A>::wf(L);
+  const float* b = m.bias + Offs<A>::bias(L);
+  const int h = lane >> 5;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const float bj = b[dreg_feature(0, h, j)];
+#pragma unroll
+    for (int t = 0; t < T; ++t) out[t][j] = bj;
+  }
+#pragma unroll
+  for (int kb = 0; kb < IN / 16; ++kb) {
+    const bf16x8 wv = w[kb * 64 + lane];
+#pragma unroll
+    for (int t = 0; t < T; ++t) out[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv, hb[t][kb], out[t], 0, 0, 0);
   }
 }
 
-// Forward pass of one wavefront (32 samples). xin: this lane's sample features, already normalized (the first D[0]
-// of them); on return y holds all P[NL] normalized outputs of this lane's sample (both lane halves agree).
+// Exchanges the upper 32 lanes of a with the lower 32 of b: {a.low, b.low} and {a.high, b.high} (v_permlane32_swap_b32).
+__device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+
+// Forward pass of one wavefront over 64 samples, lane = sample, as two 32-sample tiles (samples 0-31 and 32-63). xin: this
+// lane's sample features, already normalized (the first D[0] of them); on return y[0 .. 16) holds this lane's normalized
+// outputs. One lane per sample outside the network, so nothing around it (features, the check of the outputs, the plain
+// fallback) runs twice, as it did with each sample on both lane halves of a 32-sample wavefront.
 template <class A>
 __device__ __forceinline__ void mlp_forward_wave(const MlpDev& m, const float* xin, float* y, int lane) {
   static_assert(A::NL == 3 || A::NL == 4, "three or four layers");
-  static_assert(A::P[0] == 16 && A::P[A::NL] == 32, "one input block and one output tile");
-  const int h = lane >> 5;
-  bf16x8 h0[1];
+  static_assert(A::P[0] == 16 && A::P[A::NL] == 32 && A::D[0] <= 16 && A::D[A::NL] <= 16, "one input block, half an output tile");
+  // a tile's operand holds features 0-7 of its samples in the lower lanes and 8-15 in the upper ones
+  union Block {
+    bf16x8 v;
+    uint32_t w[4];
+  } t0, t1;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {  // lane half h takes features 8 h .. 8 h + 7 (compile-time indices only)
-    const float v0 = i < A::D[0] ? xin[i] : 0.0f;
-    const float v1 = 8 + i < A::D[0] ? xin[(8 + i) % A::D[0]] : 0.0f;
-    h0[0][i] = (__bf16)(h ? v1 : v0);
+  for (int i = 0; i < 8; ++i) {
+    t0.v[i] = (__bf16)(i < A::D[0] ? xin[i] : 0.0f);
+    t1.v[i] = (__bf16)(8 + i < A::D[0] ? xin[(8 + i) % A::D[0]] : 0.0f);
   }
-  bf16x8 h1[A::P[1] / 16];
-  mlp_layer_gelu<A, 0>(m, h0, h1, lane);
-  f32x16 out[1];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) swap_halves(t0.w[i], t1.w[i]);
+  const bf16x8 h0[2][1] = {{t0.v}, {t1.v}};
+  bf16x8 h1[2][A::P[1] / 16], h2[2][A::P[2] / 16];
+  f32x16 out[2];
+  mlp_layer_gelu<A, 0, 2>(m, h0, h1, lane);
+  mlp_layer_gelu<A, 1, 2>(m, h1, h2, lane);
   if constexpr (A::NL == 3) {
-    bf16x8 h2[A::P[2] / 16];
-    mlp_layer_gelu<A, 1>(m, h1, h2, lane);
-    mlp_layer<A, 2>(m, h2, out, lane);
+    mlp_layer_out<A, 2>(m, h2, out, lane);
   } else {
-    bf16x8 h2[A::P[2] / 16], h3[A::P[3] / 16];
-    mlp_layer_gelu<A, 1>(m, h1, h2, lane);
-    mlp_layer_gelu<A, 2>(m, h2, h3, lane);
-    mlp_layer<A, 3>(m, h3, out, lane);
+    bf16x8 h3[2][A::P[3] / 16];
+    mlp_layer_gelu<A, 2, 2>(m, h2, h3, lane);
+    mlp_layer_out<A, 2>(m, h3, out, lane);
   }
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const float mine = out[0][j], other = __shfl_xor(mine, 32);
-    y[dreg_feature(0, 0, j)] = h ? other : mine;
-    y[dreg_feature(0, 1, j)] = h ? mine : other;
+  for (int j = 0; j < 8; ++j) {  // features 0-15: lane halves 0 and 1 of the tiles' D registers
+    uint32_t a = __float_as_uint(out[0][j]), b = __float_as_uint(out[1][j]);
+    swap_halves(a, b);
+    y[dreg_feature(0, 0, j)] = __uint_as_float(a);
+    y[dreg_feature(0, 1, j)] = __uint_as_float(b);
   }
 }
 
