@@ -388,6 +388,7 @@ int fecx_create(fecx_ctx** out, int device) {
       HIPCHK(hipHostMalloc((void**)&ctx->flag_host, sizeof(int), hipHostMallocDefault));
       *ctx->flag_host = 0;
       HIPCHK(hipHostMalloc((void**)&ctx->cg_done_host, sizeof(int), hipHostMallocDefault));
+      HIPCHK(hipHostMalloc((void**)&ctx->sg_loss_host, sizeof(double), hipHostMallocDefault));
       // the allocation-free entry point's per-device scratch address, looked up once per device, device current
       require(fecx::noalloc_setup(device) == FECX_OK, FECX_ERR_HIP, "scratch symbol lookup failed");
     }
@@ -407,6 +408,7 @@ int fecx_destroy(fecx_ctx* ctx) {
   if (ctx->stream2) (void)hipStreamDestroy(ctx->stream2);
   if (ctx->flag_host) (void)hipHostFree(ctx->flag_host);
   if (ctx->cg_done_host) (void)hipHostFree(ctx->cg_done_host);
+  if (ctx->sg_loss_host) (void)hipHostFree(ctx->sg_loss_host);
   delete ctx;
   return FECX_OK;
 }

@@ -305,6 +305,7 @@ struct fecx_ctx {
   bool flag_dirty = false;
   // conjugate gradients: pinned convergence word and the events that mark the enqueued batches of iterations
   int* cg_done_host = nullptr;
+  double* sg_loss_host = nullptr;  // pinned word the loss of a gradient pass is stored to
   std::vector<hipEvent_t> cg_events;
   // profiling
   bool profiling = false;

@@ -43,111 +43,209 @@ __device__ __forceinline__ void normalized_features(const MlpDev& m, const float
   for (int f = 0; f < Feat<ARCH>::NF; ++f) x[f] = (x[f] - m.in_shift[f]) / m.in_scale[f];
 }
 
-// ------------------------------------------------------------------ training: fused forward + backward per wavefront
-template <int ARCH>
-__global__ __launch_bounds__(256) void mlp_train_kernel(TrainArgs a) {
+// ------------------------------------------------------------------ training: fused forward + backward
+// One work-group per 32 TT samples, one wavefront per 32 features of the hidden layers: wavefront w computes D tile w of every
+// layer for the TT sample tiles, and the activations go round through LDS as the next layer's B operands (two buffers, one
+// barrier per layer). The output layer, the loss and its gradient are one wavefront's work per sample tile. Every sum has
+// the order it has with one wavefront per tile.
+// The weight gradients want the same numbers with the samples as the reduction index: ds_read_tr turns the 32 x 32 tiles round
+// on their way out of LDS, so h and dz are stored as ready MFMA operands, one kilobyte per store.
+// Bound by latency on small batches (a chain of 2 NL - 1 layers) and by the write of h and dz (2.2 KB per neo-Hookean sample) on
+// large ones. With one wavefront per 32 samples doing all layers (512 wavefronts for 16,384 samples, 1.4 KB of scratch each,
+// 2-byte stores, GELU' through memory) the neo-Hookean kernel took 183 us at 16,384 samples, now 17; 97 us at 100,000.
+typedef short s16x4 __attribute__((__vector_size__(4 * sizeof(short))));
+
+template <class A>
+constexpr int train_waves() {
+  static_assert(A::P[1] == max_hidden<A>() && A::P[2] == max_hidden<A>() && A::P[A::NL - 1] == max_hidden<A>(),
+                "hidden layers of one width: one D tile per wavefront");
+  return max_hidden<A>() / 32;
+}
+
+// Operand u (samples 16 u .. 16 u + 15) of one 32-feature x 32-sample tile with k = sample: lane l, element i = feature l % 32 of
+// sample 16 u + 8 (l / 32) + i. `b` holds the tile's two B operands (k = feature). ds_read_tr16_b64, measured: in a group of 16
+// lanes, lane p element e = element p % 4 of the 8 bytes that lane 4 e + p / 4 points at; so lane c points at sample c / 4 and
+// the four features 4 (c % 4) of its group's 16. In the hidden layers' order (PERM) four features lie at block f / 16, lane
+// half f / 4 % 2, half-operand f / 8 % 2; the network's inputs are in plain order and fill one block.
+template <bool PERM>
+__device__ __forceinline__ bf16x8 transposed_operand(const bf16x8 (*b)[64], int u, int lane) {
+  union {
+    bf16x8 v;
+    s16x4 q[2];
+  } o;
+  const int c4 = lane % 4, fh = lane / 16 % 2;
+  const int kb = PERM ? fh : 0, hh = PERM ? c4 % 2 : c4 / 2, half = PERM ? c4 / 2 : c4 % 2;
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int smp = 16 * u + 8 * (lane / 32) + 4 * r + lane % 16 / 4;
+    const __bf16* p = reinterpret_cast<const __bf16*>(&b[kb][hh * 32 + smp]) + 4 * half;
+    o.q[r] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
+  }
+  return o.v;
+}
+
+template <int ARCH, int TT>
+__global__ __launch_bounds__(train_waves<Arch<ARCH>>() * 64) void mlp_train_kernel(TrainArgs a) {
   using A = Arch<ARCH>;
   using O = Offs<A>;
-  constexpr int NL = A::NL, DOUT = A::D[NL];
-  constexpr int MAXW = max_hidden<A>();
+  constexpr int NL = A::NL, DOUT = A::D[NL], W = max_hidden<A>(), NW = train_waves<A>();
+  static_assert(TT <= NW, "one wavefront per sample tile at the ends");
+  __shared__ bf16x8 act[2][TT][W / 16][64];
   const int lane = threadIdx.x % 64, h = lane >> 5;
-  const int64_t tile = (int64_t)blockIdx.x * 4 + threadIdx.x / 64;  // 32 samples per wavefront
-  const int64_t s = tile * 32 + lane % 32;
-  if (tile * 32 >= a.npad) return;  // whole wavefront out of range (npad is a multiple of 128: never taken)
-  const bool valid = s < a.n;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int64_t tile0 = (int64_t)blockIdx.x * TT;
+  const int64_t nsb = a.npad / 16;  // operands (16 samples each) per 32 features
+  const int64_t s = (tile0 + wv) * 32 + lane % 32;  // this wavefront's samples at the ends (wv < TT)
+  const bool valid = wv < TT && s < a.n;
   const int64_t row = valid ? (a.idx ? (int64_t)a.idx[s] : s) : 0;
-  float raw[Feat<ARCH>::IN_W], x[16];
+  bf16x8* hbuf = reinterpret_cast<bf16x8*>(a.hbuf);
+  bf16x8* dzbuf = reinterpret_cast<bf16x8*>(a.dzbuf);
+  if (wv < TT) {
+    float raw[Feat<ARCH>::IN_W], x[16];
 #pragma unroll
-  for (int i = 0; i < Feat<ARCH>::IN_W; ++i) raw[i] = valid ? a.X[row * Feat<ARCH>::IN_W + i] : 0.0f;
-  normalized_features<ARCH>(a.m, raw, x);
-  if (!valid) {
+    for (int i = 0; i < Feat<ARCH>::IN_W; ++i) raw[i] = valid ? a.X[row * Feat<ARCH>::IN_W + i] : 0.0f;
+    normalized_features<ARCH>(a.m, raw, x);
+    bf16x8 v;
 #pragma unroll
-    for (int f = 0; f < 16; ++f) x[f] = 0.0f;
-  }
-  bf16x8 hb[MAXW / 16];
-  f32x16 acc[MAXW / 32];
-  // h_0: rows 8h .. 8h+7 from this lane half, rows 16 + 8h .. 23 + 8h zero
-  __bf16* h0 = a.hbuf;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float v0 = i < A::D[0] ? x[i] : 0.0f;
-    const float v1 = 8 + i < A::D[0] ? x[(8 + i) % A::D[0]] : 0.0f;
-    hb[0][i] = (__bf16)(h ? v1 : v0);
-    h0[(int64_t)(8 * h + i) * a.npad + s] = hb[0][i];
-    h0[(int64_t)(16 + 8 * h + i) * a.npad + s] = (__bf16)0.0f;
-  }
-  // forward, keeping GELU'(z) per hidden layer
-  int64_t hoff = (int64_t)O::hrows(0) * a.npad, gpoff = 0;
-  auto hidden = [&](auto LC) {
-    constexpr int L = decltype(LC)::value;  // hidden layer index 1 .. NL-1
-    constexpr int W = A::P[L];
-    __bf16* hl = a.hbuf + hoff;
-    __bf16* gp = a.gpbuf + gpoff + tile * (W / 2) * 64;  // [tile][register r = 16 mt + j][lane]
-#pragma unroll
-    for (int mt = 0; mt < W / 32; ++mt)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const float z = acc[mt][j];
-        const float g = gelu(z);
-        gp[(mt * 16 + j) * 64 + lane] = (__bf16)gelu_prime(z);
-        hl[(int64_t)dreg_feature(mt, h, j) * a.npad + s] = (__bf16)g;
-        hb[2 * mt + j / 8][j % 8] = (__bf16)g;
-      }
-    hoff += (int64_t)W * a.npad;
-    gpoff += (int64_t)(a.npad / 32) * (W / 2) * 64;
-  };
-  mlp_layer<A, 0>(a.m, hb, acc, lane);
-  hidden(std::integral_constant<int, 1>());
-  mlp_layer<A, 1>(a.m, hb, acc, lane);
-  if constexpr (NL >= 3) {
-    hidden(std::integral_constant<int, 2>());
-    mlp_layer<A, 2>(a.m, hb, acc, lane);
-  }
-  if constexpr (NL >= 4) {
-    hidden(std::integral_constant<int, 3>());
-    mlp_layer<A, 3>(a.m, hb, acc, lane);
-  }
-  // loss and output gradient, dz_NL = 2 (y - t) / (n * DOUT)
-  const float gscale = 2.0f / (float)((double)a.n * DOUT);
-  double lsum = 0.0;
-  int64_t dzoff = 0;
-  for (int l = 1; l < NL; ++l) dzoff += (int64_t)A::P[l] * a.npad;
-  __bf16* dzl = a.dzbuf + dzoff;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int o = dreg_feature(0, h, j);
-    float dy = 0.0f;
-    if (valid && o < DOUT) {
-      const float t = (a.T[row * DOUT + o] - a.m.out_shift[o]) / a.m.out_scale[o];
-      const float d = acc[0][j] - t;
-      lsum += (double)d * d;
-      dy = gscale * d;
+    for (int i = 0; i < 8; ++i) {
+      const float v0 = i < A::D[0] ? x[i] : 0.0f;
+      const float v1 = 8 + i < A::D[0] ? x[(8 + i) % A::D[0]] : 0.0f;
+      v[i] = (__bf16)(valid ? (h ? v1 : v0) : 0.0f);
     }
-    acc[0][j] = dy;
-    dzl[(int64_t)o * a.npad + s] = (__bf16)dy;
+    act[0][wv][0][lane] = v;
   }
-  // wave sum of the loss, in a fixed order
+  f32x16 acc[TT];
+  bf16x8 gp[NL - 1][TT][2];  // GELU'(z) of this wavefront's features
+  int p = 0;                 // buffer of the current layer's inputs
+  int64_t ho = 0;            // operands of the layers before
+  // the inputs of layer L, from buffer p; the weights are on their way before the barrier
+  auto layer = [&](auto LC) {
+    constexpr int L = decltype(LC)::value, IN = A::P[L];
+    const int mt = L == NL - 1 ? 0 : wv;
+    const bf16x8* w = a.m.wf + O::wf(L) + (int64_t)mt * (IN / 16) * 64 + lane;
+    const float* b = a.m.bias + O::bias(L);
+    bf16x8 wr[IN / 16];
+    if (L < NL - 1 || wv < TT) {
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) lsum += __shfl_xor(lsum, off);
-  if (lane == 0) a.loss_part[tile] = lsum / ((double)a.n * DOUT);
-  // backward
-  pack_tiles<32>(acc, hb);
-  auto back = [&](auto LC) {
-    constexpr int L = decltype(LC)::value;  // dh_L = W_L^T dz_{L+1}; dz_L = dh_L * GELU'(z_L)
-    constexpr int W = A::P[L];
-    mlp_layer_t<A, L>(a.m, hb, acc, lane);
-    gpoff -= (int64_t)(a.npad / 32) * (W / 2) * 64;
-    dzoff -= (int64_t)W * a.npad;
-    const __bf16* gp = a.gpbuf + gpoff + tile * (W / 2) * 64;
-    __bf16* dz = a.dzbuf + dzoff;
+      for (int kb = 0; kb < IN / 16; ++kb) wr[kb] = w[kb * 64];
+    }
+    __syncthreads();
+    if constexpr (L == 0) {  // h_0: rows 16 .. 31 are zero
+      if (wv < TT) {
 #pragma unroll
-    for (int mt = 0; mt < W / 32; ++mt)
+        for (int u = 0; u < 2; ++u) {
+          const bf16x8 v = transposed_operand<false>(act[0][wv], u, lane), z = {};
+          hbuf[((tile0 + wv) * 2 + u) * 64 + lane] = lane / 16 % 2 ? z : v;
+        }
+      }
+      ho += nsb * 64;
+    } else {
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          hbuf[ho + (wv * nsb + (tile0 + t) * 2 + u) * 64 + lane] = transposed_operand<true>(&act[p][t][2 * wv], u, lane);
+      ho += NW * nsb * 64;
+    }
+    if constexpr (L < NL - 1) {
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        const float d = acc[mt][j] * (float)gp[(mt * 16 + j) * 64 + lane];
-        dz[(int64_t)dreg_feature(mt, h, j) * a.npad + s] = (__bf16)d;
-        hb[2 * mt + j / 8][j % 8] = (__bf16)d;
+        const float bj = b[dreg_feature(mt, h, j)];
+#pragma unroll
+        for (int t = 0; t < TT; ++t) acc[t][j] = bj;
       }
+#pragma unroll
+      for (int kb = 0; kb < IN / 16; ++kb)
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+          acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wr[kb], act[p][t][kb][lane], acc[t], 0, 0, 0);
+      p ^= 1;
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          bf16x8 v;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const float z = acc[t][8 * u + i];
+            gp[L][t][u][i] = (__bf16)gelu_prime(z);
+            v[i] = (__bf16)gelu(z);
+          }
+          act[p][t][2 * wv + u][lane] = v;
+        }
+    } else if (wv < TT) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) acc[0][j] = b[dreg_feature(0, h, j)];
+#pragma unroll
+      for (int kb = 0; kb < IN / 16; ++kb)
+        acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wr[kb], act[p][wv][kb][lane], acc[0], 0, 0, 0);
+    }
+  };
+  layer(std::integral_constant<int, 0>());
+  layer(std::integral_constant<int, 1>());
+  if constexpr (NL >= 3) layer(std::integral_constant<int, 2>());
+  if constexpr (NL >= 4) layer(std::integral_constant<int, 3>());
+  // loss and output gradient, dz_NL = 2 (y - t) / (n * DOUT)
+  int64_t dzo = (int64_t)(NL - 1) * NW * nsb * 64;
+  p ^= 1;
+  if (wv < TT) {
+    const float gscale = 2.0f / (float)((double)a.n * DOUT);
+    double lsum = 0.0;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int o = dreg_feature(0, h, j);
+      float dy = 0.0f;
+      if (valid && o < DOUT) {
+        const float t = (a.T[row * DOUT + o] - a.m.out_shift[o]) / a.m.out_scale[o];
+        const float d = acc[0][j] - t;
+        lsum += (double)d * d;
+        dy = gscale * d;
+      }
+      act[p][wv][j / 8][lane][j % 8] = (__bf16)dy;
+    }
+    // wave sum of the loss, in a fixed order
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) lsum += __shfl_xor(lsum, off);
+    if (lane == 0) a.loss_part[tile0 + wv] = lsum / ((double)a.n * DOUT);
+  }
+  // dh_L = W_L^T dz_{L+1}; dz_L = dh_L * GELU'(z_L)
+  auto back = [&](auto LC) {
+    constexpr int L = decltype(LC)::value, IN = A::P[L + 1];
+    const bf16x8* w = a.m.wb + O::wb(L) + (int64_t)wv * (IN / 16) * 64 + lane;
+    bf16x8 wr[IN / 16];
+#pragma unroll
+    for (int kb = 0; kb < IN / 16; ++kb) wr[kb] = w[kb * 64];
+    __syncthreads();
+    if constexpr (L == NL - 1) {
+      if (wv < TT) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          dzbuf[dzo + ((tile0 + wv) * 2 + u) * 64 + lane] = transposed_operand<true>(&act[p][wv][0], u, lane);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < TT; ++t) acc[t] = f32x16{};
+#pragma unroll
+    for (int kb = 0; kb < IN / 16; ++kb)
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wr[kb], act[p][t][kb][lane], acc[t], 0, 0, 0);
+    p ^= 1;
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        bf16x8 v;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = (__bf16)(acc[t][8 * u + i] * (float)gp[L - 1][t][u][i]);
+        act[p][t][2 * wv + u][lane] = v;
+      }
+    dzo -= (int64_t)NW * nsb * 64;
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)  // this wavefront's own part of the buffer
+        dzbuf[dzo + (wv * nsb + (tile0 + t) * 2 + u) * 64 + lane] = transposed_operand<true>(&act[p][t][2 * wv], u, lane);
   };
   if constexpr (NL >= 4) back(std::integral_constant<int, 3>());
   if constexpr (NL >= 3) back(std::integral_constant<int, 2>());
@@ -155,55 +253,89 @@ __global__ __launch_bounds__(256) void mlp_train_kernel(TrainArgs a) {
 }
 
 // ------------------------------------------------------------------ training: weight gradients (MFMA over samples)
-// One wavefront per (layer, 32 x 32 weight tile, chunk of samples): dW[o][i] = sum_s dz_{l+1}[o][s] h_l[i][s] with
-// samples as the MFMA reduction dimension; the tiles with it == 0 also sum dz rows for the bias gradient. Partial sums
-// per chunk go to part[chunk][param]; the reduction over chunks runs in a fixed order (mlp_update_kernel).
+// One wavefront per (layer, up to 2 x 2 weight tiles of 32 x 32, chunk of samples): dW[o][i] = sum_s dz_{l+1}[o][s] h_l[i][s] with
+// samples as the MFMA reduction dimension and the operands as the training kernel stored them; the blocks of the first inputs
+// also sum dz rows for the bias gradient. Partial sums per chunk go to part[chunk][param]; the reduction over chunks runs in a
+// fixed order (mlp_update_kernel). The blocks of one chunk are launched eight apart, so that one XCD's L2 serves all of them.
+// Bound by the read of h and dz: neo-Hookean 16,384 samples 31 us with single tiles and 32-byte pieces of feature-major rows,
+// now 11; 100,000 (218 MB) 60 us.
+template <class A, int L>
+struct WGradShape {
+  static constexpr int NOT = A::P[L + 1] / 32, NIT = Offs<A>::hrows(L) / 32;
+  static constexpr int MB = NOT > 1 ? 2 : 1, NB = NIT > 1 ? 2 : 1;
+  static constexpr int BLOCKS = (NOT / MB) * (NIT / NB);
+};
 template <int ARCH>
 __global__ __launch_bounds__(64) void mlp_wgrad_kernel(WGradArgs a) {
   using A = Arch<ARCH>;
   using O = Offs<A>;
   constexpr int NL = A::NL;
   const int lane = threadIdx.x, h = lane >> 5;
-  int t = blockIdx.x;
-  const int chunk = blockIdx.y;
-  const int64_t s0 = (int64_t)chunk * a.chunk_len;
-  int64_t hoff = 0, dzoff = 0;
+  int t = blockIdx.x / 8 % a.nblocks;
+  const int chunk = blockIdx.x / (8 * a.nblocks) * 8 + blockIdx.x % 8;
+  if (chunk >= a.nchunk) return;
+  const int64_t nsb = a.npad / 16;
+  const int64_t k0 = (int64_t)chunk * (a.chunk_len / 16), k1 = min(k0 + a.chunk_len / 16, nsb);
+  int64_t ho = 0, dzo = 0;
   auto tile = [&](auto LC) {
     constexpr int L = decltype(LC)::value;
-    constexpr int NOT = A::P[L + 1] / 32, NIT = O::hrows(L) / 32;
+    using S = WGradShape<A, L>;
+    constexpr int MB = S::MB, NB = S::NB;
     if (t < 0) return;
-    if (t >= NOT * NIT) {
-      t -= NOT * NIT;
-      hoff += (int64_t)O::hrows(L) * a.npad;
-      dzoff += (int64_t)A::P[L + 1] * a.npad;
+    if (t >= S::BLOCKS) {
+      t -= S::BLOCKS;
+      ho += (int64_t)S::NIT * nsb * 64;
+      dzo += (int64_t)S::NOT * nsb * 64;
       return;
     }
-    const int ot = t / NIT, it = t % NIT;
+    const int ot = t / (S::NIT / NB) * MB, it = t % (S::NIT / NB) * NB;
     t = -1;
-    const __bf16* dz = a.dzbuf + dzoff + (int64_t)(ot * 32 + lane % 32) * a.npad;
-    const __bf16* hl = a.hbuf + hoff + (int64_t)(it * 32 + lane % 32) * a.npad;
-    f32x16 c = {};
-    float bsum = 0.0f;
-    for (int64_t k = s0; k < s0 + a.chunk_len; k += 16) {
-      const bf16x8 av = *reinterpret_cast<const bf16x8*>(dz + k + 8 * h);
-      const bf16x8 bv = *reinterpret_cast<const bf16x8*>(hl + k + 8 * h);
-      c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, c, 0, 0, 0);
-      if (it == 0) {
+    const bf16x8* dz = reinterpret_cast<const bf16x8*>(a.dzbuf) + dzo + ot * nsb * 64 + lane;
+    const bf16x8* hl = reinterpret_cast<const bf16x8*>(a.hbuf) + ho + it * nsb * 64 + lane;
+    f32x16 c[MB][NB] = {};
+    float bsum[MB] = {};
+    for (int64_t k = k0; k < k1; k += 4) {  // samples are padded to 64
+      bf16x8 av[4][MB], bv[4][NB];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) bsum += (float)av[e];
+      for (int u = 0; u < 4; ++u) {
+#pragma unroll
+        for (int m = 0; m < MB; ++m) av[u][m] = dz[(m * nsb + k + u) * 64];
+#pragma unroll
+        for (int n = 0; n < NB; ++n) bv[u][n] = hl[(n * nsb + k + u) * 64];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+          for (int n = 0; n < NB; ++n) c[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[u][m], bv[u][n], c[m][n], 0, 0, 0);
+        if (it == 0) {
+#pragma unroll
+          for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) bsum[m] += (float)av[u][m][e];
+        }
       }
     }
     float* part = a.part + (int64_t)chunk * O::params() + O::param(L);
-    const int i = it * 32 + lane % 32;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int o = dreg_feature(ot, h, j);
-      if (o < A::D[L + 1] && i < A::D[L]) part[(int64_t)o * A::D[L] + i] = c[j];
-    }
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+      for (int n = 0; n < NB; ++n) {
+        const int i = (it + n) * 32 + lane % 32;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const int o = dreg_feature(ot + m, h, j);
+          if (o < A::D[L + 1] && i < A::D[L]) part[(int64_t)o * A::D[L] + i] = c[m][n][j];
+        }
+      }
     if (it == 0) {
-      bsum += __shfl_xor(bsum, 32);
-      const int o = ot * 32 + lane % 32;
-      if (h == 0 && o < A::D[L + 1]) part[(int64_t)A::D[L + 1] * A::D[L] + o] = bsum;
+#pragma unroll
+      for (int m = 0; m < MB; ++m) {
+        bsum[m] += __shfl_xor(bsum[m], 32);
+        const int o = (ot + m) * 32 + lane % 32;
+        if (h == 0 && o < A::D[L + 1]) part[(int64_t)A::D[L + 1] * A::D[L] + o] = bsum[m];
+      }
     }
   };
   tile(std::integral_constant<int, 0>());
@@ -213,10 +345,10 @@ __global__ __launch_bounds__(64) void mlp_wgrad_kernel(WGradArgs a) {
 }
 
 template <int ARCH>
-int wgrad_tiles() {
+int wgrad_blocks() {
   using A = Arch<ARCH>;
-  int n = 0;
-  for (int l = 0; l < A::NL; ++l) n += (A::P[l + 1] / 32) * (Offs<A>::hrows(l) / 32);
+  int n = WGradShape<A, 0>::BLOCKS + WGradShape<A, 1>::BLOCKS + WGradShape<A, 2>::BLOCKS;
+  if constexpr (A::NL >= 4) n += WGradShape<A, 3>::BLOCKS;
   return n;
 }
 
@@ -251,14 +383,33 @@ __device__ void repack_param(const MlpPack& pk, int64_t p, float w) {
   }
 }
 
+// The last work-group sums the n loss partials by one wavefront in a fixed order (lane l takes partials l, l + 64, ..., then a
+// fixed xor tree across lanes), so every run gives the same bits. The chunks of a parameter are added in ascending order with
+// eight loads on their way (64 chunks of the neo-Hookean network: 14 us one load at a time, now 5).
 template <int ARCH>
 __global__ void mlp_update_kernel(UpdateArgs a) {
+  if (a.loss && blockIdx.x == gridDim.x - 1) {
+    if (threadIdx.x >= 64) return;
+    double s = 0.0;
+    for (int64_t i = threadIdx.x; i < a.nloss; i += 64) s += a.loss_part[i];
+    for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off);
+    if (threadIdx.x == 0) a.loss[0] = s;
+    return;
+  }
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= a.np) return;
   float w = a.w[p];
   if (a.part) {
     float g = 0.0f;
-    for (int c = 0; c < a.nchunk; ++c) g += a.part[(int64_t)c * a.np + p];
+    int c = 0;
+    for (; c + 8 <= a.nchunk; c += 8) {
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = a.part[(int64_t)(c + k) * a.np + p];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) g += v[k];
+    }
+    for (; c < a.nchunk; ++c) g += a.part[(int64_t)c * a.np + p];
     if (a.grad) a.grad[p] = g;
     if (a.adam) {
       const float m1 = a.b1 * a.m1[p] + (1.0f - a.b1) * g;
@@ -270,15 +421,6 @@ __global__ void mlp_update_kernel(UpdateArgs a) {
     }
   }
   if (a.repack) repack_param<ARCH>(a.pk, p, w);
-}
-
-// Sum of the n loss partials by one wavefront in a fixed order (lane l takes partials l, l + 64, ..., then a fixed
-// xor tree across lanes), so every run gives the same bits.
-__global__ void loss_sum_kernel(const double* part, int64_t n, double* out) {
-  double s = 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += 64) s += part[i];
-  for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off);
-  if (threadIdx.x == 0) out[0] = s;
 }
 
 __global__ void gather_rows_kernel(int64_t n, int w, const int32_t* idx, const float* src, float* dst) {
@@ -635,14 +777,25 @@ __global__ void j2_feature_rows_kernel(const float* in, int64_t n, float* x) {
 }
 
 // ------------------------------------------------------------------ host launchers
+template <int ARCH, int TT>
+static void launch_train_tiles(const TrainArgs& a, hipStream_t s) {
+  static_assert(TRAIN_PAD % (32 * TT) == 0, "whole work-groups");
+  mlp_train_kernel<ARCH, TT><<<(unsigned)(a.npad / (32 * TT)), train_waves<Arch<ARCH>>() * 64, 0, s>>>(a);
+}
+// Sample tiles of one work-group: two share every weight operand, one is the shorter chain and leaves the 128-wide network,
+// with three hidden layers' GELU' in registers, two work-groups on a CU. Measured, one | two tiles, whole gradient: neo-Hookean
+// 1,500 samples 35.5 | 38.0 us, 16,384 51.6 | 47.1, 100,000 202 | 183; J2 1,500 32.8 | 36.7, 16,384 42.0 | 45.0, 100,000
+// 141 | 165. So the 256-wide network takes two once every CU (256 of them) has a work-group of one.
 template <int ARCH>
 static void launch_train(const TrainArgs& a, hipStream_t s) {
-  mlp_train_kernel<ARCH><<<(unsigned)(a.npad / 128), 256, 0, s>>>(a);
+  constexpr int MOST = max_hidden<Arch<ARCH>>() > 128 ? 2 : 1;
+  if (a.npad > 32 * 256) launch_train_tiles<ARCH, MOST>(a, s);
+  else launch_train_tiles<ARCH, 1>(a, s);
 }
 template <int ARCH>
-static void launch_wgrad(const WGradArgs& a, hipStream_t s) {
-  dim3 g((unsigned)wgrad_tiles<ARCH>(), (unsigned)a.nchunk);
-  mlp_wgrad_kernel<ARCH><<<g, 64, 0, s>>>(a);
+static void launch_wgrad(WGradArgs a, hipStream_t s) {
+  a.nblocks = wgrad_blocks<ARCH>();
+  mlp_wgrad_kernel<ARCH><<<(unsigned)((a.nchunk + 7) / 8 * 8 * a.nblocks), 64, 0, s>>>(a);
 }
 
 void mlp_launch_train(int arch, const TrainArgs& a, hipStream_t s) {
@@ -654,12 +807,9 @@ void mlp_launch_wgrad(int arch, const WGradArgs& a, hipStream_t s) {
   else launch_wgrad<FECX_MLP_NH>(a, s);
 }
 void mlp_launch_update(int arch, const UpdateArgs& a, hipStream_t s) {
-  const unsigned g = (unsigned)((a.np + 255) / 256);
+  const unsigned g = (unsigned)((a.np + 255) / 256) + (a.loss ? 1u : 0u);
   if (arch == FECX_MLP_J2) mlp_update_kernel<FECX_MLP_J2><<<g, 256, 0, s>>>(a);
   else mlp_update_kernel<FECX_MLP_NH><<<g, 256, 0, s>>>(a);
-}
-void mlp_launch_loss_sum(const double* part, int64_t n, double* out, hipStream_t s) {
-  loss_sum_kernel<<<1, 64, 0, s>>>(part, n, out);
 }
 void mlp_launch_gather(int64_t n, int w, const int32_t* idx, const float* src, float* dst, hipStream_t s) {
   if (n > 0) gather_rows_kernel<<<(unsigned)((n * w + 255) / 256), 256, 0, s>>>(n, w, idx, src, dst);
@@ -706,7 +856,6 @@ static ArchInfo make_info() {
   r.wf_vecs = O::wf_total();
   r.wb_vecs = O::wb_total();
   r.nbias = O::bias_total();
-  r.wgrad_tiles = wgrad_tiles<ARCH>();
   return r;
 }
 

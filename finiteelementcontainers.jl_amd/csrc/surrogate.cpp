@@ -68,20 +68,22 @@ void repack(fecx_ctx* ctx) {
   HIPCHK(hipGetLastError());
 }
 
-int64_t npad_of(int64_t n) { return (n + 255) / 256 * 256; }
+int64_t npad_of(int64_t n) { return (n + fecx::TRAIN_PAD - 1) / fecx::TRAIN_PAD * fecx::TRAIN_PAD; }
 
 // One forward + backward pass over n samples (rows idx[0..n) of X/T, or 0..n); the summed gradient goes to `grad`
-// (optional) and, with adam, into an Adam step. The mean loss is written to the device double *loss.
+// (optional) and, with adam, into an Adam step. The mean loss is written to *loss, which the device can reach.
 void grad_pass(fecx_ctx* ctx, const float* X, const float* T, const int32_t* idx, int64_t n, float* grad, bool adam,
                float lr, double* loss) {
   const int arch = ctx->sg_arch;
   const fecx::ArchInfo ai = fecx::arch_info(arch);
   const int64_t npad = npad_of(n);
-  int64_t hrows = 32, dzrows = 0, gprows = 0;
-  for (int l = 1; l < ai.nl; ++l) { hrows += ai.p[l]; gprows += ai.p[l]; }
+  int64_t hrows = 32, dzrows = 0;
+  for (int l = 1; l < ai.nl; ++l) hrows += ai.p[l];
   for (int l = 1; l <= ai.nl; ++l) dzrows += ai.p[l];
-  const int chunk_len = 256;
-  const int nchunk = (int)(npad / chunk_len);
+  // At most 64 chunks of the samples: enough wavefronts for the chip (12 or 24 per chunk), a bounded size of their partial
+  // sums, and the shortest chunks that allows.
+  const int64_t chunk_len = (npad + 64 * fecx::TRAIN_PAD - 1) / (64 * fecx::TRAIN_PAD) * fecx::TRAIN_PAD;
+  const int nchunk = (int)((npad + chunk_len - 1) / chunk_len);
   fecx::TrainArgs ta{};
   ta.m = mlp_dev(ctx);
   ta.n = n;
@@ -91,7 +93,6 @@ void grad_pass(fecx_ctx* ctx, const float* X, const float* T, const int32_t* idx
   ta.idx = idx;
   ta.hbuf = (__bf16*)dev_atleast(ctx, "sg_h", sizeof(__bf16) * hrows * npad);
   ta.dzbuf = (__bf16*)dev_atleast(ctx, "sg_dz", sizeof(__bf16) * dzrows * npad);
-  ta.gpbuf = (__bf16*)dev_atleast(ctx, "sg_gp", sizeof(__bf16) * gprows * npad);
   ta.loss_part = (double*)dev_atleast(ctx, "sg_lossp", sizeof(double) * (npad / 32));
   fecx::mlp_launch_train(arch, ta, ctx->stream);
   HIPCHK(hipGetLastError());
@@ -107,6 +108,9 @@ void grad_pass(fecx_ctx* ctx, const float* X, const float* T, const int32_t* idx
   fecx::UpdateArgs u = update_args(ctx);
   u.part = wa.part;
   u.nchunk = nchunk;
+  u.loss_part = ta.loss_part;
+  u.nloss = npad / 32;
+  u.loss = loss;
   u.grad = grad;
   if (adam) {
     ctx->sg_step += 1;
@@ -117,8 +121,6 @@ void grad_pass(fecx_ctx* ctx, const float* X, const float* T, const int32_t* idx
     u.c2 = (float)(1.0 / (1.0 - std::pow(0.999, (double)ctx->sg_step)));
   }
   fecx::mlp_launch_update(arch, u, ctx->stream);
-  HIPCHK(hipGetLastError());
-  fecx::mlp_launch_loss_sum(ta.loss_part, npad / 32, loss, ctx->stream);
   HIPCHK(hipGetLastError());
 }
 
@@ -299,10 +301,9 @@ int fecx_surrogate_gradient(fecx_ctx* ctx, const float* X, const float* T, int64
     require_net(ctx);
     require(X && T && n > 0 && grad, FECX_ERR_ARG, "bad arrays");
     require(n <= (int64_t(1) << 30), FECX_ERR_ARG, "too many samples for one pass");
-    double* dl = (double*)dev_atleast(ctx, "sg_loss", sizeof(double));
-    grad_pass(ctx, X, T, nullptr, n, grad, false, 0.0f, dl);
+    grad_pass(ctx, X, T, nullptr, n, grad, false, 0.0f, ctx->sg_loss_host);
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    if (loss) HIPCHK(hipMemcpy(loss, dl, sizeof(double), hipMemcpyDeviceToHost));
+    if (loss) *loss = *(volatile double*)ctx->sg_loss_host;
   });
 }
 

@@ -14,15 +14,17 @@ struct MlpPack {  // writable views of the packed weights
   float* bias;
 };
 
+constexpr int64_t TRAIN_PAD = 64;  // samples of one training work-group and one step of the weight gradients
+
 struct TrainArgs {
   MlpDev m;
-  int64_t n, npad;       // samples in the batch, padded count (multiple of 256)
+  int64_t n, npad;       // samples in the batch, padded count (multiple of TRAIN_PAD)
   const float* X;        // raw inputs, rows idx[s] (or s)
   const float* T;        // raw targets
   const int32_t* idx;    // optional row map of the batch
-  __bf16* hbuf;          // h_l, l < NL: hrows(l) x npad (feature-major)
-  __bf16* dzbuf;         // dz_l, 1 <= l <= NL: P[l] x npad
-  __bf16* gpbuf;         // GELU'(z_l), 1 <= l < NL: [tile][register][lane]
+  __bf16* hbuf;          // h_l, l < NL: [32 features of hrows(l)][16 samples of npad][lane][8], lane l element i = feature
+                         // l % 32 of sample 8 (l / 32) + i
+  __bf16* dzbuf;         // dz_l, 1 <= l <= NL: the same for P[l] features
   double* loss_part;     // npad / 32
 };
 
@@ -30,7 +32,9 @@ struct WGradArgs {
   const __bf16* hbuf;
   const __bf16* dzbuf;
   int64_t npad;
-  int nchunk, chunk_len;  // nchunk * chunk_len == npad
+  int nchunk;
+  int64_t chunk_len;      // a multiple of TRAIN_PAD; the last chunk ends at npad
+  int nblocks;            // set by the launcher
   float* part;            // nchunk x nparams
 };
 
@@ -39,6 +43,9 @@ struct UpdateArgs {
   float* w;               // canonical FP32 parameters
   const float* part;      // chunk partial gradients, or nullptr (repack only)
   int nchunk;
+  const double* loss_part;  // loss partials to sum into *loss, or nullptr
+  int64_t nloss;
+  double* loss;
   float* grad;            // optional: summed gradient out
   int adam, repack;
   float* m1;
@@ -69,7 +76,6 @@ struct MatBatchArgs {
 void mlp_launch_train(int arch, const TrainArgs& a, hipStream_t s);
 void mlp_launch_wgrad(int arch, const WGradArgs& a, hipStream_t s);
 void mlp_launch_update(int arch, const UpdateArgs& a, hipStream_t s);
-void mlp_launch_loss_sum(const double* part, int64_t n, double* out, hipStream_t s);
 void mlp_launch_gather(int64_t n, int w, const int32_t* idx, const float* src, float* dst, hipStream_t s);
 void mlp_launch_forward(int arch, const MatBatchArgs& a, hipStream_t s);
 void mlp_launch_material(int arch, bool surrogate, const MatBatchArgs& a, hipStream_t s);
@@ -89,7 +95,6 @@ struct ArchInfo {
   int in_w, nfeat, out_w;
   int64_t nparams, wf_vecs, wb_vecs;
   int nbias;
-  int wgrad_tiles;
 };
 ArchInfo arch_info(int arch);
 
