@@ -107,6 +107,17 @@ fecx::ReduceArgs reduce_args(fecx_ctx* ctx) {
   return r;
 }
 
+fecx::FusedArgs fused_args(fecx_ctx* ctx, int mode, double* R, double* vals) {
+  fecx::FusedArgs fa{};
+  fa.nx = ctx->snx; fa.ny = ctx->sny; fa.nz = ctx->snz;
+  fa.epos = get<int32_t>(ctx, "epos");
+  fa.nodeinfo = get<int2>(ctx, "nodeinfo");
+  fa.rmap = ctx->partial ? get<int32_t>(ctx, "rmap") : nullptr;
+  fa.vals = (mode & fecx::MODE_K) ? vals : nullptr;
+  fa.R = (mode & fecx::MODE_R) ? R : nullptr;
+  return fa;
+}
+
 // Number of pipeline chunks of a matrix assembly. One by default: on MI355X the overlapped pieces measured slower
 // than back-to-back launches (hex8 neo-Hookean 96^3: 2.04 ms one piece, 2.15-2.38 ms with 4-32 pieces), the two
 // kernels competing for the same CU resources.
@@ -170,8 +181,8 @@ bool build_nodeinfo(fecx_ctx* ctx) {
 
 // The scatter design a matrix assembly takes (FECX_SCATTER_*): the fused kernel for residual + Jacobian (or Jacobian)
 // assemblies of a one-block structured hex8 mesh with a plain material when asked for, or by default for the
-// vector-valued materials (on the scalar Poisson problem the two-phase path is faster: its element work is cheap and
-// the fused kernel's halo recompute and one-work-group-per-CU marching do not pay); the atomic and coloured designs
+// vector-valued materials (on the scalar Poisson problem the two-phase path is faster, with one lane per element and per
+// row on large meshes: its element work is cheap and the fused kernel's halo recompute and marching do not pay); the atomic and coloured designs
 // only where they are built (structured hex8, Poisson or neo-Hookean) and never for the allocation-free entry point
 // (their zero fill is a memset); the two-phase path everywhere else.
 int scatter_path(fecx_ctx* ctx, int mode, bool surrogate, bool noalloc) {
@@ -225,6 +236,10 @@ void assemble(fecx_ctx* ctx, int mode, const double* U, const double* V, double*
   const bool surrogate = surrogate_phys && ctx->sg_enabled;
   float *kel = get<float>(ctx, "Kel"), *rel = get<float>(ctx, "Rel");
   const int path = scatter_path(ctx, mode, surrogate_phys, noalloc);
+  // a structured scalar mesh assembled whole: one lane per element and per row
+  bool lanes = path == FECX_SCATTER_TWO_PHASE && ctx->structured && ctx->nf == 1 && ctx->mp.phys == FECX_POISSON &&
+               ctx->block_mp.size() == 1 && (mode == fecx::MODE_K || mode == (fecx::MODE_R | fecx::MODE_K)) &&
+               (noalloc || pipeline_chunks(ctx, mode) == 1) && fecx::poisson_hex8_applies(ctx->ne);
   if (noalloc) require(!surrogate, FECX_ERR_UNSUPPORTED, "the allocation-free entry point does not run surrogate materials");
   if (noalloc && path == FECX_SCATTER_TWO_PHASE) {  // the fused kernel keeps no element-private outputs
     const size_t kb = sizeof(float) * (size_t)ctx->ne * ctx->pairs.npairs * ctx->nf * ctx->nf;
@@ -235,8 +250,12 @@ void assemble(fecx_ctx* ctx, int mode, const double* U, const double* V, double*
             "holds at most " + std::to_string(fecx::NOALLOC_SCRATCH_BYTES) + " (use fecx_assemble_vector_matrix)");
     unsigned char* base = (unsigned char*)fecx::noalloc_scratch(ctx->device);
     require(base != nullptr, FECX_ERR_STATE, "no scratch address for this device");
+    // one lane per element pads the elements to 64; a mesh that only just fits keeps the other kernels
+    const size_t kp = sizeof(float) * (size_t)fecx::poisson_hex8_words(ctx->ne, ctx->pairs.npairs);
+    const size_t rp = sizeof(float) * (size_t)fecx::poisson_hex8_words(ctx->ne, ctx->nnpe);
+    lanes = lanes && kp + rp <= fecx::NOALLOC_SCRATCH_BYTES;
     kel = (float*)base;
-    rel = (float*)(base + kb_al);
+    rel = (float*)(base + (lanes ? kp : kb_al));
   }
   Prof prof(ctx);
   if (noalloc) prof.ctx = nullptr;  // no HIP events
@@ -261,13 +280,7 @@ void assemble(fecx_ctx* ctx, int mode, const double* U, const double* V, double*
     HIPCHK(hipGetLastError());
   }
   if (path != FECX_SCATTER_TWO_PHASE) {
-    fecx::FusedArgs fa{};
-    fa.nx = ctx->snx; fa.ny = ctx->sny; fa.nz = ctx->snz;
-    fa.epos = get<int32_t>(ctx, "epos");
-    fa.nodeinfo = get<int2>(ctx, "nodeinfo");
-    fa.rmap = ctx->partial ? get<int32_t>(ctx, "rmap") : nullptr;
-    fa.vals = (mode & fecx::MODE_K) ? vals : nullptr;
-    fa.R = (mode & fecx::MODE_R) ? R : nullptr;
+    const fecx::FusedArgs fa = fused_args(ctx, mode, R, vals);
     int rc = 0;
     if (path == FECX_SCATTER_FUSED) {
       prof.run("fused", ctx->stream, [&] { rc = fecx::launch_fused_hex8(ctx->nf, ea, fa, ctx->stream); });
@@ -280,6 +293,17 @@ void assemble(fecx_ctx* ctx, int mode, const double* U, const double* V, double*
       });
     }
     require(rc == 0, FECX_ERR_UNSUPPORTED, "no kernel of this scatter design for this nf / physics");
+    HIPCHK(hipGetLastError());
+    const int hflag = read_flag(ctx);
+    prof.finish();
+    require(hflag == 0, FECX_ERR_NUMERIC, "element kernel met a non-positive Jacobian determinant or a NaN");
+    return;
+  }
+  if (lanes) {
+    const fecx::FusedArgs fa = fused_args(ctx, mode, R, vals);
+    prof.run("element", ctx->stream, [&] { fecx::launch_poisson_hex8_elements(mode, ea, fa, ctx->stream); });
+    HIPCHK(hipGetLastError());
+    prof.run("reduce", ctx->stream, [&] { fecx::launch_poisson_hex8_rows(mode, ea, fa, ctx->stream); });
     HIPCHK(hipGetLastError());
     const int hflag = read_flag(ctx);
     prof.finish();
@@ -667,8 +691,9 @@ int fecx_build_pattern(fecx_ctx* ctx, int64_t* nnz) {
           off1[(size_t)la * nnpe + b] = (int16_t)fecx::pair_pos(nnpe, la, b, fecx::pair_ref(nnpe, la, b).slot);
       upload(ctx, "kel_off1", off1);
     }
-    dev(ctx, "Rel", sizeof(float) * ctx->ne * ctx->nnpe * nf);
-    dev(ctx, "Kel", sizeof(float) * ctx->ne * ctx->pairs.npairs * nf * nf);
+    // room for the elements padded to 64 (poisson_hex8_words)
+    dev(ctx, "Rel", sizeof(float) * (ctx->ne + 63) * ctx->nnpe * nf);
+    dev(ctx, "Kel", sizeof(float) * (ctx->ne + 63) * ctx->pairs.npairs * nf * nf);
     if (detect_structured_hex8(ctx) && ctx->device >= 0 && !build_nodeinfo(ctx)) ctx->structured = false;
     ctx->has_pattern = true;
     if (nnz) *nnz = ctx->nnz;

@@ -169,6 +169,12 @@ struct FusedArgs {
 };
 // returns 0, or -1 if the (nf, phys) combination has no fused kernel (or the mesh exceeds 2^31 tile planes)
 int launch_fused_hex8(int nf, const ElementArgs& a, const FusedArgs& f, hipStream_t s);
+// The two-phase assembly of a structured scalar hex8 mesh with one lane per element and per row (poisson_hex8.hip): whether a mesh of
+// ne elements takes it, the words it keeps for nw words per element, and its two kernels. mode: MODE_K or MODE_R | MODE_K.
+bool poisson_hex8_applies(int64_t ne);
+int64_t poisson_hex8_words(int64_t ne, int nw);
+void launch_poisson_hex8_elements(int mode, const ElementArgs& a, const FusedArgs& f, hipStream_t s);
+void launch_poisson_hex8_rows(int mode, const ElementArgs& a, const FusedArgs& f, hipStream_t s);
 // the atomic (scatter 1) and coloured (scatter 2) designs on structured hex8 meshes; vals and R zero-filled first
 int launch_scatter_hex8(int nf, int scatter, const ElementArgs& a, const FusedArgs& f, hipStream_t s);
 // returns 0, or -1 if the (kind, nf) combination has no mass kernel; rho multiplies every weight

@@ -9,7 +9,8 @@
 // Vector: the same groups sum the node's incident element rows into the residual field (the atomic scatter of
 // src/assemblers/Assemblers.jl:72-87 restated as an owner-computes gather).
 // These kernels share this contract (launch_buckets routes the light rows, then the heavy ones):
-//   reduce_scalar_hex8_kernel   scalar hex8 light rows: lanes add their words into LDS slot accumulators;
+//   reduce_scalar_hex8_kernel   scalar hex8 light rows: lanes add their words into LDS slot accumulators (large structured
+//                               Poisson meshes: ph_row_kernel, poisson_hex8.hip, one lane per row);
 //   reduce_scatter_kernel       light rows of up to 32 blocks of 2 and 3 fields and of scalar tet10, and the tet10 heavy rows
 //                               (scalar and 3-field) of up to 72 blocks: the same scatter, 16, 32 or 64 lanes per row;
 //   reduce_merged_kernel        3-field tet10 meshes whose rows have at most 65 blocks: both buckets of
