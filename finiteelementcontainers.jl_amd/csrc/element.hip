@@ -1338,6 +1338,7 @@ static void launch_tet10(int mode, const ElementArgs& a, hipStream_t s) {
 
 int launch_element(int kind, int nf, int mode, const ElementArgs& a, hipStream_t s) {
   const int phys = a.mp.phys;
+  if (launch_lane_element(kind, nf, mode, a, s) == 0) return 0;
   if (nf == 1 && phys == FECX_POISSON) {
     if (kind == FECX_QUAD4) { launch_modes<FECX_QUAD4, 1, FECX_POISSON>(mode, a, s); return 0; }
     if (kind == FECX_HEX8) { launch_modes<FECX_HEX8, 1, FECX_POISSON>(mode, a, s); return 0; }

@@ -157,6 +157,9 @@ struct ElementArgs {
 // returns 0, or -1 if the (kind, nf, phys) combination has no kernel
 int launch_element(int kind, int nf, int mode, const ElementArgs& a, hipStream_t s);
 
+// the same for the calls that lane_element.hip's kernels are faster on, or -1 (launch_element asks it first)
+int launch_lane_element(int kind, int nf, int mode, const ElementArgs& a, hipStream_t s);
+
 // Fused residual + CSR assembly of a structured hex8 mesh (element.hip, fused_hex8_kernel).
 struct FusedArgs {
   int nx, ny, nz;                // node counts per direction

@@ -278,10 +278,12 @@ struct Mat<FECX_NEOHOOKEAN> {
   __device__ static void eval(const MatParams& mp, const R* H, const float*, float*, R* P, float* C, bool& bad) {
     const R lam = mp.p[0], mu = mp.p[1];
     const R tr = H[0] + H[4] + H[8];
-    const R trH2 = H[0] * H[0] + H[4] * H[4] + H[8] * H[8] + R(2) * (H[1] * H[3] + H[2] * H[6] + H[5] * H[7]);
-    const R detH = H[0] * (H[4] * H[8] - H[5] * H[7]) - H[1] * (H[3] * H[8] - H[5] * H[6]) +
-                   H[2] * (H[3] * H[7] - H[4] * H[6]);
-    const R Jm1 = tr + R(0.5) * (tr * tr - trH2) + detH;
+    // Sums of products are written as the fused multiply-adds they are, so that every kernel rounds them alike: left to the
+    // compiler, which product of a sum is fused depends on the code around it.
+    const R trH2 = fma(R(2), fma(H[5], H[7], fma(H[1], H[3], H[2] * H[6])), fma(H[8], H[8], fma(H[0], H[0], H[4] * H[4])));
+    const R c0 = fma(H[4], H[8], -(H[5] * H[7])), c1 = fma(H[3], H[8], -(H[5] * H[6])), c2 = fma(-H[4], H[6], H[3] * H[7]);
+    const R detH = fma(H[2], c2, fma(H[0], c0, -(H[1] * c1)));
+    const R Jm1 = fma(R(0.5), fma(tr, tr, -trH2), tr) + detH;
     const R J = R(1) + Jm1;
     if (!(J > R(0))) bad = true;
     R lnJ;
@@ -290,18 +292,18 @@ struct Mat<FECX_NEOHOOKEAN> {
     const R F[9] = {1 + H[0], H[1], H[2], H[3], 1 + H[4], H[5], H[6], H[7], 1 + H[8]};
     const R iJ = R(1) / J;
     R FiT[9];  // cofactor(F) / J
-    FiT[0] = (F[4] * F[8] - F[5] * F[7]) * iJ; FiT[1] = (F[5] * F[6] - F[3] * F[8]) * iJ;
-    FiT[2] = (F[3] * F[7] - F[4] * F[6]) * iJ; FiT[3] = (F[2] * F[7] - F[1] * F[8]) * iJ;
-    FiT[4] = (F[0] * F[8] - F[2] * F[6]) * iJ; FiT[5] = (F[1] * F[6] - F[0] * F[7]) * iJ;
-    FiT[6] = (F[1] * F[5] - F[2] * F[4]) * iJ; FiT[7] = (F[2] * F[3] - F[0] * F[5]) * iJ;
-    FiT[8] = (F[0] * F[4] - F[1] * F[3]) * iJ;
+    FiT[0] = fma(F[4], F[8], -(F[5] * F[7])) * iJ; FiT[1] = fma(-F[3], F[8], F[5] * F[6]) * iJ;
+    FiT[2] = fma(-F[4], F[6], F[3] * F[7]) * iJ; FiT[3] = fma(F[2], F[7], -(F[1] * F[8])) * iJ;
+    FiT[4] = fma(F[0], F[8], -(F[2] * F[6])) * iJ; FiT[5] = fma(F[1], F[6], -(F[0] * F[7])) * iJ;
+    FiT[6] = fma(F[1], F[5], -(F[2] * F[4])) * iJ; FiT[7] = fma(F[2], F[3], -(F[0] * F[5])) * iJ;
+    FiT[8] = fma(F[0], F[4], -(F[1] * F[3])) * iJ;
     if (P) {
 #pragma unroll
       for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-          const R htf = H[0 * 3 + i] * FiT[0 * 3 + j] + H[1 * 3 + i] * FiT[1 * 3 + j] + H[2 * 3 + i] * FiT[2 * 3 + j];
-          P[i * 3 + j] = mu * (H[i * 3 + j] + htf) + lam * lnJ * FiT[i * 3 + j];
+          const R htf = fma(H[2 * 3 + i], FiT[2 * 3 + j], fma(H[0 * 3 + i], FiT[0 * 3 + j], H[1 * 3 + i] * FiT[1 * 3 + j]));
+          P[i * 3 + j] = fma(mu, H[i * 3 + j] + htf, lam * lnJ * FiT[i * 3 + j]);
         }
     }
     if (C) {
@@ -362,16 +364,17 @@ struct Mat<FECX_NEOHOOKEAN> {
 #pragma unroll
     for (int l = 0; l < 3; ++l)
 #pragma unroll
-      for (int j = 0; j < 3; ++j) M[l * 3 + j] = Gv[0 * 3 + l] * C[0 * 3 + j] + Gv[1 * 3 + l] * C[1 * 3 + j] + Gv[2 * 3 + l] * C[2 * 3 + j];
+      for (int j = 0; j < 3; ++j) M[l * 3 + j] = fmaf(Gv[2 * 3 + l], C[2 * 3 + j], fmaf(Gv[0 * 3 + l], C[0 * 3 + j], Gv[1 * 3 + l] * C[1 * 3 + j]));
     float tr = 0;
 #pragma unroll
     for (int i = 0; i < 9; ++i) tr += C[i] * Gv[i];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
-      for (int j = 0; j < 3; ++j)
-        out[i * 3 + j] = mu * Gv[i * 3 + j] + c1 * (C[i * 3 + 0] * M[0 * 3 + j] + C[i * 3 + 1] * M[1 * 3 + j] + C[i * 3 + 2] * M[2 * 3 + j]) +
-                         lam * tr * C[i * 3 + j];
+      for (int j = 0; j < 3; ++j) {
+        const float s = fmaf(C[i * 3 + 2], M[2 * 3 + j], fmaf(C[i * 3 + 0], M[0 * 3 + j], C[i * 3 + 1] * M[1 * 3 + j]));
+        out[i * 3 + j] = fmaf(lam * tr, C[i * 3 + j], fmaf(mu, Gv[i * 3 + j], c1 * s));
+      }
   }
 };
 
