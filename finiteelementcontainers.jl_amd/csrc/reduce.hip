@@ -18,7 +18,7 @@
 //   reduce_rows_kernel          slot-owner lanes for everything else: light scalar quad4 rows, heavy hex8/quad4 rows and
 //                               tet10 rows of more than 72 blocks;
 //   reduce_expand_kernel        mass matrices of 2 or 3 fields, from one word per node pair (blocks m I);
-//   reduce_vector_kernel / reduce_vector_group_kernel   calls without CSR values (one thread, or 16 lanes, per row).
+//   reduce_vector_kernel / reduce_vector_tet10_kernel   calls without CSR values (one thread, or on tet10 vertices 16 lanes, per row).
 // All sum a slot's (or a row's) contributions in ascending incidence order, so every form gives the same bits.
 #include <algorithm>
 #include <type_traits>
@@ -672,9 +672,7 @@ static int launch_buckets(const ReduceArgs& a, hipStream_t s) {
 // element rows into R in ascending incidence order -- the order of the matrix kernel's residual sum, so the two give
 // the same bits. Incidences go in batches of 8: indices first, then all their loads, then the FP64 adds.
 template <int NF>
-__global__ __launch_bounds__(256) void reduce_vector_kernel(ReduceArgs a) {
-  const int64_t pos = a.p0 + xcd_chunk(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
-  if (pos >= a.p1) return;
+__device__ __forceinline__ void vector_row(const ReduceArgs& a, int64_t pos) {
   const int4 ri = a.rowinfo[pos];
   const int64_t n = ri.x;
   const int32_t c0 = ri.y, ninc = ri.w & 0xFFFF;
@@ -717,20 +715,25 @@ __global__ __launch_bounds__(256) void reduce_vector_kernel(ReduceArgs a) {
 #pragma unroll
   for (int i = 0; i < NF; ++i) a.R[n * NF + i] = acc[i];
 }
+template <int NF>
+__global__ __launch_bounds__(256) void reduce_vector_kernel(ReduceArgs a) {
+  const int64_t pos = a.p0 + xcd_chunk(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+  if (pos < a.p1) vector_row<NF>(a, pos);
+}
 
 // Vector-only reduction with G lanes per row, for rows with many incidences (tet10 vertices: 24): lane l loads the
 // incidences l, l + G, ... of each pass of CHV, all before any add, stages their element rows in LDS, and lane i < NF
 // of the row then adds component i of incidences 0, 1, ... in ascending order: the order, and so the bits, of the
 // thread-per-row kernel above and of the matrix kernel's residual sum.
 template <int NF, int G, int CHV>
-__global__ __launch_bounds__(256) void reduce_vector_group_kernel(ReduceArgs a) {
+__device__ __forceinline__ void vector_group(const ReduceArgs& a, int64_t p0, int64_t p1) {  // rows [p0, min(p0 + 256 / G, p1))
   constexpr int RPW = 256 / G, PER = CHV / G;
   static_assert(CHV % G == 0, "whole incidences per lane");
   __shared__ float s_r[RPW][CHV][NF];
   __shared__ int s_maxpass;
   const int lane = threadIdx.x % G, grp = threadIdx.x / G;
-  const int64_t pos = a.p0 + xcd_chunk(blockIdx.x, gridDim.x) * RPW + grp;
-  const bool valid = pos < a.p1;
+  const int64_t pos = p0 + grp;
+  const bool valid = pos < p1;
   const int4 ri = valid ? a.rowinfo[pos] : make_int4(0, 0, 0, 0);
   const int32_t c0 = ri.y, ninc = ri.w & 0xFFFF;
   if (threadIdx.x == 0) s_maxpass = 0;
@@ -766,6 +769,23 @@ __global__ __launch_bounds__(256) void reduce_vector_group_kernel(ReduceArgs a) 
   if (valid && lane < NF) a.R[(int64_t)ri.x * NF + lane] = acc;
 }
 
+// tet10: the vertex rows (24 incidences, 16 lanes each, 32 incidences staged per pass: 0.370 ms against 0.393 with 8 lanes and
+// 24, and 0.414 with 4, on tet10 80^3 x 6) and, behind them in the same launch, the light rows (edge midpoints, at most 8
+// incidences: one batch of loads) one thread each. heavy: work-groups of the vertex rows, a multiple of 8 like the others (XCD
+// ranges). Bound by the latency of the incidence list and the scattered rows behind it; two launches one after the other
+// (the light ones first) took 2 to 4 us longer: residuals 33 x 39 x 35 x 6 75.9 against 73.7 us, 25^3 x 6 46.7 against 42.7, 12^3 x 6
+// 33.4 against 29.4. Mixing the two along the rows gives 71.4, 44.2 and 29.6.
+constexpr int VEC_G = 16;
+template <int NF>
+__global__ __launch_bounds__(256) void reduce_vector_tet10_kernel(ReduceArgs a, int64_t split, unsigned heavy) {
+  if (blockIdx.x < heavy) {
+    vector_group<NF, VEC_G, 32>(a, split + xcd_chunk(blockIdx.x, heavy) * (256 / VEC_G), a.p1);
+  } else {
+    const int64_t pos = a.p0 + xcd_chunk(blockIdx.x - heavy, gridDim.x - heavy) * 256 + threadIdx.x;
+    if (pos < split) vector_row<NF>(a, pos);
+  }
+}
+
 int launch_reduce_expand(int nf, const ReduceArgs& a, hipStream_t s) {
   if (a.p1 <= a.p0 || !a.vals) return 0;
   auto go = [&](auto part) {
@@ -783,26 +803,12 @@ int launch_reduce(int nf, const ReduceArgs& a, hipStream_t s) {
   if (!a.vals) {
     if (!a.R) return 0;
     if (a.nnpe == 10) {
-      // light rows (edge midpoints, at most 8 incidences: one batch of loads) one thread each, then the vertex rows
-      // (24 incidences) 16 lanes each, 32 incidences staged per pass (0.370 ms against 0.393 with 8 lanes and 24, and
-      // 0.414 with 4, on tet10 80^3 x 6)
-      ReduceArgs lo = a, hi = a;
-      lo.p1 = std::min(a.p1, std::max(a.p0, a.nlight));
-      hi.p0 = std::max(a.p0, a.nlight);
       if (nf != 1 && nf != 3) return -1;
-      if (lo.p1 > lo.p0) {
-        int64_t grid = (lo.p1 - lo.p0 + 255) / 256;
-        grid = (grid + 7) / 8 * 8;  // XCD remap needs a multiple of 8
-        if (nf == 1) reduce_vector_kernel<1><<<(unsigned)grid, 256, 0, s>>>(lo);
-        else reduce_vector_kernel<3><<<(unsigned)grid, 256, 0, s>>>(lo);
-      }
-      if (hi.p1 > hi.p0) {
-        constexpr int G = 16;
-        int64_t grid = (hi.p1 - hi.p0 + 256 / G - 1) / (256 / G);
-        grid = (grid + 7) / 8 * 8;
-        if (nf == 1) reduce_vector_group_kernel<1, G, 32><<<(unsigned)grid, 256, 0, s>>>(hi);
-        else reduce_vector_group_kernel<3, G, 32><<<(unsigned)grid, 256, 0, s>>>(hi);
-      }
+      const int64_t split = std::min(a.p1, std::max(a.p0, a.nlight));  // light rows [p0, split), vertex rows [split, p1)
+      const auto groups = [](int64_t rows, int per) { return (unsigned)(((rows + per - 1) / per + 7) / 8 * 8); };
+      const unsigned heavy = groups(a.p1 - split, 256 / VEC_G), grid = heavy + groups(split - a.p0, 256);
+      if (nf == 1) reduce_vector_tet10_kernel<1><<<grid, 256, 0, s>>>(a, split, heavy);
+      else reduce_vector_tet10_kernel<3><<<grid, 256, 0, s>>>(a, split, heavy);
       return 0;
     }
     int64_t grid = (a.p1 - a.p0 + 255) / 256;
