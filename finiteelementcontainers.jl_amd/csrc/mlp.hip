@@ -672,23 +672,55 @@ __global__ __launch_bounds__(256) void material_kernel(MatBatchArgs a) {
 }
 
 // ------------------------------------------------------------------ network-only forward (raw units)
-template <int ARCH>
-__global__ __launch_bounds__(256) void mlp_forward_kernel(MatBatchArgs a) {
+// TT = 2: 64 samples per wavefront, lane = sample, as in the update. TT = 1: 32, on both lane halves; the lower
+// stores. One tile is the shorter chain, two load every weight once for both and go further
+// where there is work for them; the J2 network's two tiles at 3 wavefronts per SIMD (40 bytes of scratch) beat 2. One tile | two
+// without | with that cap: J2 3,000 samples 25.0 | 28.0 | 35.6 us, 100,000 44.1 | 43.3 | 45.4, 2,000,000 422 | 445 | 360;
+// neo-Hookean (no cap: it spills) 3,000 40.2 | 31.7, 100,000 69.6 | 50.9, 2,000,000 669 | 566.
+template <int ARCH, int TT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ARCH == FECX_MLP_J2 && TT == 2 ? 3 : 1, 8)))
+void mlp_forward_kernel(MatBatchArgs a) {
   using A = Arch<ARCH>;
   using FT = Feat<ARCH>;
+  constexpr int SPW = 32 * TT;  // samples per wavefront
   const int lane = threadIdx.x % 64;
-  const int64_t tile = (int64_t)blockIdx.x * 4 + threadIdx.x / 64;  // 64 samples per wavefront
-  const int64_t i = tile * 64 + lane;
-  if (tile * 64 >= a.n) return;
+  const int64_t tile = (int64_t)blockIdx.x * 4 + threadIdx.x / 64;
+  const int64_t i = tile * SPW + lane % SPW;
+  if (tile * SPW >= a.n) return;
   const bool valid = i < a.n;
-  float raw[16] = {}, x[16], yn[16];
+  float raw[16] = {}, x[16];
 #pragma unroll
   for (int c = 0; c < FT::IN_W; ++c) raw[c] = valid ? a.in[i * FT::IN_W + c] : 0.0f;
   normalized_features<ARCH>(a.m, raw, x);
-  mlp_forward_wave<A>(a.m, x, yn, lane);
-  if (valid) {
+  if constexpr (TT == 2) {
+    float yn[16];
+    mlp_forward_wave<A>(a.m, x, yn, lane);
+    if (valid) {
 #pragma unroll
-    for (int o = 0; o < FT::OUT_W; ++o) a.out[i * FT::OUT_W + o] = yn[o] * a.m.out_scale[o] + a.m.out_shift[o];
+      for (int o = 0; o < FT::OUT_W; ++o) a.out[i * FT::OUT_W + o] = yn[o] * a.m.out_scale[o] + a.m.out_shift[o];
+    }
+  } else {
+    const int h = lane >> 5;
+    bf16x8 h0[1][1];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const float lo = k < A::D[0] ? x[k] : 0.0f, hi = 8 + k < A::D[0] ? x[(8 + k) % A::D[0]] : 0.0f;
+      h0[0][0][k] = (__bf16)(h ? hi : lo);
+    }
+    f32x16 out[1];
+    mlp_hidden<A, 1>(a.m, h0, out, lane);
+    float yn[16];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {  // the halves' D registers to both
+      uint32_t lo = __float_as_uint(out[0][j]), hi = lo;
+      swap_halves(lo, hi);
+      yn[dreg_feature(0, 0, j)] = __uint_as_float(lo);
+      yn[dreg_feature(0, 1, j)] = __uint_as_float(hi);
+    }
+    if (valid && h == 0) {
+#pragma unroll
+      for (int o = 0; o < FT::OUT_W; ++o) a.out[i * FT::OUT_W + o] = yn[o] * a.m.out_scale[o] + a.m.out_shift[o];
+    }
   }
 }
 
@@ -815,10 +847,12 @@ void mlp_launch_gather(int64_t n, int w, const int32_t* idx, const float* src, f
   if (n > 0) gather_rows_kernel<<<(unsigned)((n * w + 255) / 256), 256, 0, s>>>(n, w, idx, src, dst);
 }
 void mlp_launch_forward(int arch, const MatBatchArgs& a, hipStream_t s) {
-  const unsigned g = (unsigned)((a.n + 255) / 256);
   if (a.n == 0) return;
-  if (arch == FECX_MLP_J2) mlp_forward_kernel<FECX_MLP_J2><<<g, 256, 0, s>>>(a);
-  else mlp_forward_kernel<FECX_MLP_NH><<<g, 256, 0, s>>>(a);
+  const bool one = arch == FECX_MLP_J2 && a.n <= (1 << 18);  // 140,000 samples 51 | 55 us, 280,000 77.6 | 77.4
+  const unsigned g = one ? (unsigned)((a.n + 127) / 128) : (unsigned)((a.n + 255) / 256);
+  if (one) mlp_forward_kernel<FECX_MLP_J2, 1><<<g, 256, 0, s>>>(a);
+  else if (arch == FECX_MLP_J2) mlp_forward_kernel<FECX_MLP_J2, 2><<<g, 256, 0, s>>>(a);
+  else mlp_forward_kernel<FECX_MLP_NH, 2><<<g, 256, 0, s>>>(a);
 }
 void mlp_launch_material(int arch, bool surrogate, const MatBatchArgs& a, hipStream_t s) {
   const unsigned g = (unsigned)((a.n + 255) / 256);

@@ -220,6 +220,22 @@ __device__ __forceinline__ void mlp_layer_out(const MlpDev& m, const bf16x8 (&hb
   }
 }
 
+// all layers of T tiles, from their input operands to the output layer's D tiles
+template <class A, int T>
+__device__ __forceinline__ void mlp_hidden(const MlpDev& m, const bf16x8 (&h0)[T][1], f32x16 (&out)[T], int lane) {
+  static_assert(A::NL == 3 || A::NL == 4, "three or four layers");
+  bf16x8 h1[T][A::P[1] / 16], h2[T][A::P[2] / 16];
+  mlp_layer_gelu<A, 0, T>(m, h0, h1, lane);
+  mlp_layer_gelu<A, 1, T>(m, h1, h2, lane);
+  if constexpr (A::NL == 3) {
+    mlp_layer_out<A, T>(m, h2, out, lane);
+  } else {
+    bf16x8 h3[T][A::P[3] / 16];
+    mlp_layer_gelu<A, 2, T>(m, h2, h3, lane);
+    mlp_layer_out<A, T>(m, h3, out, lane);
+  }
+}
+
 // Exchanges the upper 32 lanes of a with the lower 32 of b: {a.low, b.low} and {a.high, b.high} (v_permlane32_swap_b32).
 __device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
   const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
@@ -233,7 +249,6 @@ __device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
 // fallback) runs twice, as it did with each sample on both lane halves of a 32-sample wavefront.
 template <class A>
 __device__ __forceinline__ void mlp_forward_wave(const MlpDev& m, const float* xin, float* y, int lane) {
-  static_assert(A::NL == 3 || A::NL == 4, "three or four layers");
   static_assert(A::P[0] == 16 && A::P[A::NL] == 32 && A::D[0] <= 16 && A::D[A::NL] <= 16, "one input block, half an output tile");
   // a tile's operand holds features 0-7 of its samples in the lower lanes and 8-15 in the upper ones
   union Block {

@@ -43,3 +43,7 @@ def test_inference_at_tile_edges(fec, mlpref, gpu, arch):
         assert torch.equal(net.forward(X[:n].contiguous()), full[:n]), n
         assert torch.equal(fec.surrogate.material_update(asm, kind, Xs[:n].contiguous()), update[:n]), n
         assert net.fallbacks() == (n, n)
+    # the longest batch that runs with one tile per wavefront and the shortest with two: the same bits per sample
+    big = X.repeat((1 << 18) // len(X) + 2, 1)
+    for n in ((1 << 18) - 3, (1 << 18) + 1):
+        assert torch.equal(net.forward(big[:n].contiguous()), full.repeat(len(big) // len(X), 1)[:n]), n
