@@ -20,7 +20,7 @@
  *    stream (fecx_set_stream). Assembly calls return after the stream is synchronised,
  *    so results can be read at once (the reference's callers read them immediately,
  *    src/Solvers.jl:128-153) and a folded element is reported by that call. The DOF
- *    plumbing calls (fecx_update_field_*, fecx_extract_field_unknowns) only enqueue:
+ *    plumbing calls (fecx_update_field*, fecx_extract_field_unknowns) only enqueue:
  *    work ordered on the same stream sees their results.
  */
 #ifndef FECX_H
