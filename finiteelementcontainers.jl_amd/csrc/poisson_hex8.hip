@@ -125,8 +125,9 @@ __device__ __forceinline__ void ph_element(const MatParams& mp, const PhNode (&n
 }
 
 constexpr int PH_ELEMS = 256;  // elements of one work-group
-// Bound by VALU issue, some 3,000 instructions per element: 128^3 elements 164 us (8 lanes per element: 295). STREAM: nontemporal stores, where the words of the mesh do not fit the 256 MB Infinity Cache anyway (128^3 step 357
-// against 382 us, 121 x 117 x 128 307 against 332; below, the rows read them from there: 64^3 62 against 69 us).
+// Bound by VALU issue, some 3,000 instructions per element: 128^3 elements 164 us (8 lanes per element: 295). STREAM: nontemporal
+// stores, where the words of the mesh do not fit the 256 MB Infinity Cache anyway (128^3 step 357 against 382 us, 121 x 117 x 128
+// 307 against 332; below, the rows read them from there: 64^3 62 against 69 us).
 template <bool DO_R, bool STREAM>
 __global__ __launch_bounds__(PH_ELEMS) void ph_element_kernel(ElementArgs a, FusedArgs f) {
   const uint32_t nex = f.nx - 1, ney = f.ny - 1;
@@ -163,8 +164,8 @@ __global__ __launch_bounds__(PH_ELEMS) void ph_element_kernel(ElementArgs a, Fus
 // consecutive in the CSR, so they are packed in LDS and stored as one range, in whole 128-byte lines but for its ends. Bound by
 // that traffic: 128^3 elements, 369 MB read and 464 MB written in about 185 us (reduce_scalar_hex8_kernel, 8 lanes per row with
 // an LDS read-add-write per word: 347). ROWS per work-group: 64 fills the chip sooner, 256 walks the words in longer
-// pieces: 64^3 step 61.5 against 64.2 us, 101 x 83 x 127 205 against 194. (Backwards, from the elements stored
-// last: as fast as this on large meshes, 32^3 37.0 against 34.8 us.)
+// pieces: 64^3 step 61.5 against 64.2 us, 101 x 83 x 127 205 against 194. (Backwards, from the elements stored last: as fast
+// on large meshes, 32^3 37.0 against 34.8 us.)
 template <bool DO_R, int ROWS>
 __global__ __launch_bounds__(ROWS) void ph_row_kernel(ElementArgs a, FusedArgs f) {
   __shared__ __attribute__((aligned(16))) double all_rows[ROWS / 64][64 * 27 + 2];

@@ -469,25 +469,42 @@ __device__ __forceinline__ void scatter_rows(const ReduceArgs& a, int64_t first,
     const CsrRow row = csr_row(a.vals, PART ? a.rmap : nullptr, __builtin_amdgcn_readlane(ri.z, rw * LPR), NFO * NFO);
     double* dst = row.vals;
     const int before = PART && row.map ? 0 : (int)((reinterpret_cast<uintptr_t>(dst) >> 3) & 15);
-    for (int m = wl - before; m < NFO * w; m += 64) {
-      if (m < 0) continue;
-      double x;
+    auto word = [&](int m) -> double {
       if constexpr (NFO > NF) {
         int i = 0, c = m;  // CSR row and column: m = i w + c
 #pragma unroll
         for (int q = 1; q < NFO; ++q)
           if (m >= q * w) { i = q; c = m - q * w; }
         const int sl = c / NFO;
-        x = c - sl * NFO == i ? s_acc[g0 + rw][sl] : 0.0;
+        return c - sl * NFO == i ? s_acc[g0 + rw][sl] : 0.0;
       } else {
-        x = s_acc[g0 + rw][m];
+        return s_acc[g0 + rw][m];
       }
+    };
+    auto put = [&](int m, double x) {
       if constexpr (NFO >= 2) {
         if (!PART || !row.map) __builtin_nontemporal_store(x, dst + m);  // written once, never read here
         else if (const int q = row.map[m]; q >= 0) dst[q] = x;
       } else {
         dst[m] = x;
       }
+    };
+    if constexpr (NFO > NF && SMAX <= 32) {  // five words per lane: every LDS read issued before the stores
+      constexpr int NCH = (NFO * NFO * SMAX + 15 + 63) / 64;
+      double x[NCH];
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) {
+        const int m = wl - before + 64 * c;
+        x[c] = m >= 0 && m < NFO * w ? word(m) : 0.0;
+      }
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) {
+        const int m = wl - before + 64 * c;
+        if (m >= 0 && m < NFO * w) put(m, x[c]);
+      }
+    } else {
+      for (int m = wl - before; m < NFO * w; m += 64)
+        if (m >= 0) put(m, word(m));
     }
   }
   if (!a.R) return;
@@ -526,7 +543,9 @@ __global__ __launch_bounds__(RED_THREADS) void reduce_expand_kernel(ReduceArgs a
 }
 template <bool PART, int NNPE, int NFO>
 static int launch_expand(const ReduceArgs& a, hipStream_t s) {
-  constexpr int LPR = NNPE == 10 ? 16 : 8;
+  // 32 lanes per row (four or two incidences at once): hex8 64^3 182.9 us with 8 lanes, 175.8 with 16 or 32, 40 x 45 x 42 72.7 against
+  // 64.9, 20 x 25 x 22 31.1 against 27.3; tet10 24^3 x 6 100.5 us with 16, 99.2 with 32
+  constexpr int LPR = 32;
   ReduceArgs lo = a, hi = a;
   lo.p1 = std::min(a.p1, a.nlight);
   hi.p0 = std::max(a.p0, a.nlight);
