@@ -532,9 +532,9 @@ __global__ __launch_bounds__(RED_THREADS) void reduce_scatter_kernel(ReduceArgs 
 
 // Consistent mass of NFO fields: every block of an element matrix is m I, so the element kernel stores the one word m per
 // node pair (a ninth of the words of full 3 x 3 blocks) and the row's slots are summed as scalars and written out as
-// blocks, zeros included. Light rows take as many lanes as an element row has words (8, or 16 for tet10), heavier ones a
-// wavefront, with accumulators for the 255 blocks that a row may have. Elastic hex8 64^3 (65 million values): element
-// kernel and reduction 78 + 293 us with full blocks, 23 + 142 us with one word per pair.
+// blocks, zeros included. Light rows take 32 lanes (quad4: 8), heavier ones a wavefront, with accumulators for the 255 blocks that a row
+// may have. Elastic hex8 64^3 (65 million values): element kernel and reduction 78 + 293 us with full blocks, 23 + 142 us with
+// one word per pair on 8 lanes per row, 23 + 137 us on 32.
 template <bool PART, int NNPE, int NFO, int LPR, int CHK, int SMAX>
 __global__ __launch_bounds__(RED_THREADS) void reduce_expand_kernel(ReduceArgs a) {
   __shared__ ScatterLDS<1, NNPE, LPR, CHK, SMAX> L;
@@ -544,8 +544,9 @@ __global__ __launch_bounds__(RED_THREADS) void reduce_expand_kernel(ReduceArgs a
 template <bool PART, int NNPE, int NFO>
 static int launch_expand(const ReduceArgs& a, hipStream_t s) {
   // 32 lanes per row (four or two incidences at once): hex8 64^3 182.9 us with 8 lanes, 175.8 with 16 or 32, 40 x 45 x 42 72.7 against
-  // 64.9, 20 x 25 x 22 31.1 against 27.3; tet10 24^3 x 6 100.5 us with 16, 99.2 with 32
-  constexpr int LPR = 32;
+  // 64.9, 20 x 25 x 22 31.1 against 27.3; tet10 24^3 x 6 100.5 us with 16, 99.2 with 32; quad4, whose rows have 9 blocks, 500^2
+  // 55.9 us with 8, 79.4 with 32
+  constexpr int LPR = NNPE == 4 ? 8 : 32;
   ReduceArgs lo = a, hi = a;
   lo.p1 = std::min(a.p1, a.nlight);
   hi.p0 = std::max(a.p0, a.nlight);
