@@ -56,3 +56,19 @@ def test_rows_match_the_fused_kernel(fec, gpu, counts, fixed, source):
     asm.stiffness_storage.fill_(float("nan"))  # every value is written
     fec.assemble_stiffness_(asm, fec.stiffness, Uu, p)
     assert torch.equal(asm.stiffness_storage, out[AUTO][1])
+
+
+@pytest.mark.parametrize("counts", [(33, 34, 33), (61, 72, 66)])
+def test_allocation_free_call_gives_the_same_bits(fec, gpu, counts):
+    """The allocation-free entry point takes the same kernels, its elements padded to 64 in its own scratch."""
+    print(f"[poisson rows] allocation-free {counts}", flush=True)
+    mesh = _brick(fec, *counts)
+    V = fec.FunctionSpace(mesh, "H1Field", "Lagrange")
+    asm = fec.SparseMatrixAssembler(fec.ScalarFunction(V, "u"), sparse_matrix_type="csr", device=gpu.index or 0)
+    p = fec.create_parameters(mesh, asm, fec.Poisson("sines", 1.5))
+    Uu = torch.from_numpy(np.cos(0.37 * np.arange(asm.dof.unknown_dofs.size))).to(gpu)
+    fec.assemble_vector_and_stiffness_(asm, Uu, p)
+    R, K = torch.full_like(asm.residual_storage, float("nan")), torch.full_like(asm.stiffness_storage, float("nan"))
+    P = fec.assembler._ptr
+    asm.ctx.call("fecx_assemble_vector_matrix_noalloc", P(p.field), P(R), P(K))
+    assert torch.equal(R, asm.residual_storage) and torch.equal(K, asm.stiffness_storage)
