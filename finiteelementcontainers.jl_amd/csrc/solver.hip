@@ -106,20 +106,22 @@ struct LineShape {
 };
 template <int NF>
 struct LinePtr {
-  int64_t rb;  // first block of the line
-  int n;       // its columns (0: past the last line)
+  int64_t rb;  // first block of the line (0 where it has none)
+  int n;       // its columns (0: past the last line, or a node that no element touches)
 };
 template <int NF>
 __device__ __forceinline__ LinePtr<NF> line_ptr(const CsrView& A, uint32_t g, uint32_t lines) {
   LinePtr<NF> p{0, 0};
   if (g < lines) {
     const int64_t* q = (NF == 0 ? A.rptr : A.bptr) + g;
-    p.rb = q[0];
-    p.n = (int)(q[1] - q[0]) * LineShape<NF>::B;
+    const int64_t rb = q[0];
+    p.n = (int)(q[1] - rb) * LineShape<NF>::B;
+    p.rb = p.n > 0 ? rb : 0;  // the last rows, empty, start where the matrix ends
   }
   return p;
 }
-// this lane's columns j0 + u L of the line; a column past the line repeats one of its own (an empty line: entry 0)
+// this lane's columns j0 + u L of the line; a column past the line repeats one of its own (an empty line: the matrix's entry
+// 0, which csr_view makes sure exists)
 template <int NF>
 __device__ __forceinline__ int line_col(const LinePtr<NF>& p, int j) { return j < p.n ? j : (p.n > 0 ? p.n - 1 : 0); }
 template <int NF>
@@ -222,6 +224,10 @@ __global__ void diag_inv_kernel(CsrView A, double* dinv) {
   const int i = (int)(row - r * NF);
   const int64_t rb = A.bptr[r];
   const int deg = (int)(A.bptr[r + 1] - rb);
+  if (deg == 0) {  // a node that no element touches: no entry to read
+    dinv[row] = 1.0;
+    return;
+  }
   int lo = 0, hi = deg - 1;
   while (lo < hi) {
     const int mid = (lo + hi) / 2;
@@ -476,6 +482,12 @@ fecx::CsrView csr_view(fecx_ctx* ctx, const double* vals) {
     A.nrows = (int64_t)ctx->unknown_dofs.size();
     A.rptr = get<int64_t>(ctx, "rptr");
     A.rcol = get<int32_t>(ctx, "rcol");
+  }
+  if (ctx->nnz == 0) {  // every free node is loose: what the empty lines load in place of their columns is one zero
+    double* zero = get<double>(ctx, "sv_zero");
+    if (!zero) zero = upload(ctx, "sv_zero", std::vector<double>(1, 0.0));
+    A.vals = zero;
+    A.bcol = A.rcol = (const int32_t*)zero;
   }
   return A;
 }

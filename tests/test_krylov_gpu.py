@@ -87,3 +87,73 @@ def test_spmv_and_cg_iterations(fec, gpu, name):
         assert it.value == k
         assert np.linalg.norm(xg.cpu().numpy() - xs) <= 1e-9 * np.linalg.norm(xs)
         assert abs(res.value - np.linalg.norm(r)) <= 1e-9 * np.linalg.norm(b)
+
+
+def _loose(fec, name):
+    """(mesh, nf, fixed): a brick or square with a loose node (of no element) before, between and after the others', the last
+    rows of the matrix being empty; "alone": every node of an element is fixed, so that the matrix has no entry"""
+    m, nf, fixed = _mesh(fec, name.replace(" alone", ""))
+    n = m.num_nodes
+    at = np.concatenate([[-1], np.arange(n // 2), [-1], np.arange(n // 2, n), [-1, -1]])  # new node -> old node
+    new = np.empty(n, np.int64)
+    new[at[at >= 0]] = np.flatnonzero(at >= 0)
+    coords = np.where(at[:, None] >= 0, m.coords[at], 1.7)
+    mesh = fec.BlockMesh(coords, [("b", new[m.conn - 1] + 1)], m.element_type)
+    fixed = {d: new[nodes - 1] + 1 for d, nodes in fixed.items()}
+    if "alone" in name:
+        fixed = {d: new + 1 for d in range(nf)}
+    return mesh, nf, fixed, np.flatnonzero(at < 0)
+
+
+@pytest.mark.parametrize("name", ["hex8 3 nf1", "hex8 3", "hex8 3 roller", "quad4 5 nf2", "hex8 2 nf1 alone", "hex8 2 alone"])
+def test_rows_of_loose_nodes(fec, gpu, name):
+    """Nodes that no element touches have empty rows: a product of zero, a unit preconditioner, and an unknown that CG leaves at its
+    start (b is zero there, or the matrix has no entry). Tolerances as above."""
+    print(f"[krylov] loose nodes {name}", flush=True)
+    mesh, nf, fixed, loose = _loose(fec, name)
+    space = fec.FunctionSpace(mesh, "H1Field", "Lagrange")
+    var = fec.ScalarFunction(space, "u") if nf == 1 else fec.VectorFunction(space, "displ")
+    asm = fec.SparseMatrixAssembler(var, sparse_matrix_type="csr", device=0)
+    for d, nodes in fixed.items():
+        mesh.nodeset_nodes[f"_f{d}"] = nodes
+    bcs = [fec.DirichletBC(var.names[d], lambda X, t: 0.0, nset_name=f"_f{d}") for d in fixed]
+    physics = fec.Poisson() if nf == 1 else fec.Mechanics(fec.PlaneStrain() if nf == 2 else None)
+    p = fec.create_parameters(mesh, asm, physics, dirichlet_bcs=bcs)
+    Uu = fec.create_unknowns(asm)
+    fec.assemble_mass_(asm, fec.mass, Uu, p)
+    A = fec.mass(asm).to_scipy()
+    n = A.shape[0]
+    empty = np.isin((asm.dof.unknown_dofs - 1) // nf, loose)
+    assert np.array_equal(np.diff(A.indptr) == 0, empty) and empty[-1]
+    g = np.random.default_rng(2)
+    P = fec.assembler._ptr
+    values = fec.mass(asm).values if asm.nnz else torch.full((1,), float("nan"), dtype=torch.float64, device=gpu)
+    x, b = g.standard_normal(n), g.standard_normal(n)
+    if asm.nnz:
+        b[empty] = 0.0
+    xd, bd = torch.from_numpy(x).to(gpu), torch.from_numpy(b).to(gpu)
+    y, dinv = torch.full_like(Uu, np.nan), torch.full_like(Uu, np.nan)
+    asm.ctx.call("fecx_csr_spmv", P(values), P(xd), P(y))
+    assert np.all(np.abs(y.cpu().numpy() - A @ x) <= 500 * 2.0 ** -53 * (abs(A) @ np.abs(x)))
+    asm.ctx.call("fecx_csr_diagonal_inverse", P(values), P(dinv))
+    diag = A.diagonal()
+    assert np.array_equal(dinv.cpu().numpy(), np.where(diag != 0.0, 1.0 / np.where(diag != 0.0, diag, 1.0), 1.0))
+    for pre in (1, 0):
+        xg = xd.clone()
+        it, res = ctypes.c_int(-1), ctypes.c_double(-1.0)
+        asm.ctx.call("fecx_cg_solve", P(values), P(bd), P(xg), ctypes.c_double(1e-9), ctypes.c_double(0.0), ctypes.c_int(5),
+                     ctypes.c_int(pre), ctypes.byref(it), ctypes.byref(res))
+        d = dinv.cpu().numpy() if pre else np.ones(n)
+        xs, r = x.copy(), b - A @ x
+        q = d * r
+        rz = r @ q
+        for _ in range(5):
+            Aq = A @ q
+            a = rz / (q @ Aq) if asm.nnz else 0.0
+            xs, r = xs + a * q, r - a * Aq
+            new = r @ (d * r)
+            q, rz = d * r + new / rz * q, new
+        assert it.value == 5
+        assert np.linalg.norm(xg.cpu().numpy() - xs) <= 1e-9 * np.linalg.norm(xs)
+        assert abs(res.value - np.linalg.norm(r)) <= 1e-9 * np.linalg.norm(b)
+        assert np.array_equal(xg.cpu().numpy()[empty], x[empty])
