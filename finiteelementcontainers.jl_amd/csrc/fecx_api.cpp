@@ -598,6 +598,9 @@ int fecx_build_pattern(fecx_ctx* ctx, int64_t* nnz) {
       }
       require((int64_t)ctx->rptr.size() == (int64_t)ctx->unknown_dofs.size() + 1, FECX_ERR_STATE, "row count");
       ctx->nnz = (int64_t)ctx->rcol.size();
+      // every row complete (the split nodes belong to no element): still a list, whose presence tells the kernels that
+      // row_place counts entries
+      if (rmap.empty()) rmap.push_back(-1);
       std::vector<int32_t> rcol32(ctx->rcol.begin(), ctx->rcol.end());
       upload(ctx, "rmap", rmap);
       upload(ctx, "rptr", ctx->rptr);

@@ -57,3 +57,20 @@ def test_partial_rows_equal_unconstrained(fec, gpu, name, design):
         assert np.abs(K.data - ref.data).max() <= 1e-13 * np.abs(ref.data).max()
     else:
         assert np.array_equal(K.data, ref.data) and np.array_equal(R, R0[u])
+
+
+@pytest.mark.parametrize("name", ["quad4 6", "hex8 5", "tet10 2", "fan 32"])
+def test_split_node_of_no_element(fec, gpu, name):
+    """The only node with some fixed and some free components belongs to no element: a dof-level CSR whose rows are all complete."""
+    print(f"[partial rows] split loose node, {name}", flush=True)
+    m = _mesh(fec, name)
+    n = m.num_nodes
+    mesh = fec.BlockMesh(np.vstack([m.coords, m.coords.mean(axis=0)]), [("b", m.conn)], m.element_type)
+    _, R0, K0 = _assemble(fec, mesh, {}, AUTO)
+    asm, R, K = _assemble(fec, mesh, {1: np.array([n + 1])}, AUTO)
+    u = asm.dof.unknown_dofs - 1
+    ref = K0[u][:, u].tocsr()
+    ref.sort_indices()
+    assert K.nnz == K0.nnz and K.shape[0] == K0.shape[0] - 1
+    assert np.array_equal(K.indptr, ref.indptr) and np.array_equal(K.indices, ref.indices)
+    assert np.array_equal(K.data, ref.data) and np.array_equal(R, R0[u])
