@@ -245,7 +245,8 @@ int fecx_update_field_unknowns(fecx_ctx* ctx, const double* Uu, double* U);
 int fecx_update_field_dirichlet(fecx_ctx* ctx, const double* vals, double* U);
 
 /* _update_for_assembly! (src/Parameters.jl:404-442) in one launch: U[dirichlet_dofs] = bc (unless bc is NULL),
- * U[unknown_dofs] = Uu, and, for the actions, V[unknown_dofs] = Vu (Vu and V may be NULL). */
+ * U[unknown_dofs] = Uu, and, for the actions, V[unknown_dofs] = Vu (unless V is NULL). An array that would be read or
+ * written and is NULL is refused, here and in the other field calls. */
 int fecx_update_fields(fecx_ctx* ctx, const double* bc, const double* Uu, double* U, const double* Vu, double* V);
 
 /* Uu = U[unknown_dofs]: extract_field_unknowns! (src/DofManagers.jl:203-213). */
