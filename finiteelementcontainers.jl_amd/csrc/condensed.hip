@@ -50,7 +50,8 @@ __device__ __forceinline__ int64_t diag_pos(const int64_t* bptr, const int32_t* 
   return NF * NF * rb + (int64_t)i * NF * (bptr[r + 1] - rb) + diag_in_line<NF>(bptr, bcol, r, i);
 }
 
-// stage 1: partial[wg] = sum of the diagonal entries of the work-group's rows (in row order within a fixed tree)
+// stage 1: partial[wg] = sum of the diagonal entries of the work-group's rows (in row order within a fixed tree). A node that
+// no element touches has empty rows and adds nothing.
 template <int NF>
 __global__ __launch_bounds__(CD_THREADS) void trace_partial_kernel(int64_t nrows, const int64_t* bptr,
                                                                      const int32_t* bcol, const double* vals,
@@ -58,7 +59,7 @@ __global__ __launch_bounds__(CD_THREADS) void trace_partial_kernel(int64_t nrows
   __shared__ double sh[CD_THREADS];
   const int64_t row = (int64_t)blockIdx.x * CD_THREADS + threadIdx.x;
   double d = 0.0;
-  if (row < nrows) d = vals[diag_pos<NF>(bptr, bcol, row / NF, (int)(row % NF))];
+  if (row < nrows && bptr[row / NF + 1] > bptr[row / NF]) d = vals[diag_pos<NF>(bptr, bcol, row / NF, (int)(row % NF))];
   const double s = cd_block_sum(d, sh);
   if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }

@@ -280,3 +280,34 @@ def test_csc_matches_oracle_and_is_symmetric(fec, orc, gpu, case):
     assert e2 < TOL and em < TOL
     A = K.to_scipy()
     assert (A != A.T).nnz == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["hex8 3 nf1", "hex8 3", "quad4 5 nf2"])
+def test_penalty_with_nodes_of_no_element(fec, gpu, name):
+    """Empty rows add nothing to the trace. Its sum has at most 68 rows x 3 terms of one sign: relative error below 204 eps for
+    any order of the sum, 1e-13 with the products around it."""
+    from test_krylov_gpu import _loose
+    print(f"[condensed] loose nodes {name}", flush=True)
+    mesh, nf, _, loose = _loose(fec, name)
+    space = fec.FunctionSpace(mesh, "H1Field", "Lagrange")
+    fixed = np.array([loose[0], loose[1], loose[1] + 1, loose[-1]]) + 1  # loose nodes and one of an element
+    mesh.nodeset_nodes["_c"] = fixed
+    stiff = {}
+    for condensed in (False, True):
+        var = fec.ScalarFunction(space, "u") if nf == 1 else fec.VectorFunction(space, "displ")
+        asm = fec.SparseMatrixAssembler(var, sparse_matrix_type="csr", use_condensed=condensed, device=gpu.index or 0)
+        bcs = [fec.DirichletBC(var.names[0], lambda X, t: 0.0, nset_name="_c")] if condensed else []
+        physics = fec.Poisson() if nf == 1 else fec.Mechanics(fec.PlaneStrain() if nf == 2 else None)
+        p = fec.create_parameters(mesh, asm, physics, dirichlet_bcs=bcs)
+        fec.assemble_stiffness_(asm, fec.stiffness, fec.create_unknowns(asm), p)
+        stiff[condensed] = fec.stiffness(asm).to_scipy().tocsr()
+    ref = stiff[False].copy()
+    con = np.isin(np.arange(ref.shape[0]), nf * (fixed - 1))
+    rows = np.repeat(np.arange(ref.shape[0]), np.diff(ref.indptr))
+    penalty = 1e6 * ref.diagonal().sum() / ref.shape[0]
+    ref.data = np.where(con[rows], np.where(ref.indices == rows, penalty, 0.0), ref.data)
+    got = stiff[True]
+    assert np.array_equal(got.indptr, ref.indptr) and np.array_equal(got.indices, ref.indices)
+    assert np.abs(got.data - ref.data).max() <= 1e-13 * penalty
+    assert np.array_equal(got.data[~con[rows]], ref.data[~con[rows]])
