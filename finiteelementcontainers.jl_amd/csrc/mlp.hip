@@ -453,11 +453,20 @@ __device__ __forceinline__ void nh_plain(const MatParams& mp, const float* H, fl
 }
 
 // ------------------------------------------------------------------ surrogate decode + residual check
+// Whether all N outputs are finite: a maximum drops NaN, so the deviations below cannot tell. 0 y is NaN unless y is finite.
+template <int N>
+__device__ __forceinline__ bool all_finite(const float* y) {
+  float z = 0.0f;
+#pragma unroll
+  for (int o = 0; o < N; ++o) z = fmaf(y[o], 0.0f, z);
+  return z == 0.0f;
+}
+
 // J2: the network's {sigma, dplastic, deqps} is accepted when it satisfies the return-mapping equations to `tol`:
 //   elastic law   |sigma - (kappa tr(eps - ep_new) I + 2 mu dev(eps - ep_new))| <= tol sigma_y
 //   yield         |f| <= tol sigma_y when deqps > 0 (on the yield surface), f <= tol sigma_y otherwise
 //   flow          |dplastic - sqrt(3/2) deqps n| <= tol sigma_y / (2 mu), deqps >= -tol sigma_y / (2 mu)
-// The tangent data follow from the closed-form consistent tangent at the network's plastic multiplier.
+// and all of it is finite. The tangent data follow from the closed-form consistent tangent at the network's plastic multiplier.
 __device__ __forceinline__ bool j2_surrogate(const MatParams& mp, const float* H, const float* so, const float* y,
                                              float tol, float* P, float* sn, float* C) {
   const float E = mp.p[0], nu = mp.p[1], sy = mp.p[2], Hh = mp.p[3];
@@ -502,7 +511,7 @@ __device__ __forceinline__ bool j2_surrogate(const MatParams& mp, const float* H
 #pragma unroll
   for (int i = 0; i < 9; ++i) rf = fmaxf(rf, fabsf(dep[i] - r32 * fmaxf(dal, 0.0f) * s[i] * inv));
   r = fmaxf(r, rf / eref);
-  if (!(r <= tol)) return false;
+  if (!(r <= tol) || !all_finite<13>(y)) return false;
 #pragma unroll
   for (int i = 0; i < 9; ++i) P[i] = sig[i];
 #pragma unroll
@@ -525,7 +534,7 @@ __device__ __forceinline__ bool j2_surrogate(const MatParams& mp, const float* H
 
 // NH: the network's {P, C^-1 - I} is accepted when C C^-1 = I to `tol` and P agrees to `tol` with the stress the
 // predicted C^-1 implies, P(F, C^-1) = mu (F - F C^-1) + lambda ln J F C^-1 (F^-T = F C^-1), relative to the stress
-// scale (mu + lambda) max(|H|, 0.01).
+// scale (mu + lambda) max(|H|, 0.01), and all of it is finite.
 __device__ __forceinline__ bool nh_surrogate(const MatParams& mp, const float* H, const float* y, float tol, float* P,
                                              float* C) {
   const float lam = mp.p[0], mu = mp.p[1];
@@ -566,7 +575,7 @@ __device__ __forceinline__ bool nh_surrogate(const MatParams& mp, const float* H
     rp = fmaxf(rp, fabsf(y[i] - pp));
   }
   r = fmaxf(r, rp / ps);
-  if (!(r <= tol)) return false;
+  if (!(r <= tol) || !all_finite<15>(y)) return false;
 #pragma unroll
   for (int i = 0; i < 9; ++i) { P[i] = y[i]; C[i] = FiT[i]; }
   C[9] = mu - lam * lnJ;

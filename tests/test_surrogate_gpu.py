@@ -193,3 +193,51 @@ def test_newton_with_surrogate_reaches_plain_tolerance(fec, gpu):
     d = np.linalg.norm(out[True][0] - out[False][0]) / np.linalg.norm(out[False][0])
     print(f"[surrogate] solution difference {d:.2e}", flush=True)
     assert d < 1e-5
+
+
+@pytest.mark.parametrize("arch", [0, 1])
+def test_outputs_that_are_not_finite_fall_back(fec, gpu, arch):
+    """A sample whose network output has a NaN or an infinity is never accepted, whichever component it is in and however wide the
+    tolerance, not even where a frozen decision says so: the plain model's output (1e-6, as above), and one fallback each."""
+    print(f"[surrogate] outputs that are not finite, arch {arch}", flush=True)
+    plain_phys = fec.J2Plasticity(*J2_PROPS) if arch == 0 else fec.NeoHookean(1.0, 0.5)
+    surr_phys = fec.J2Surrogate(*J2_PROPS) if arch == 0 else fec.NeoHookeanSurrogate(1.0, 0.5)
+    kind = (fec._lib.J2_SURROGATE, fec._lib.J2) if arch == 0 else (fec._lib.NH_SURROGATE, fec._lib.NEOHOOKEAN)
+    wl, asm, p = _asm(fec, gpu, surr_phys)
+    net = fec.Surrogate(asm, arch, seed=5)
+    net.set_tolerance(1e30)
+    w = net.params()
+    g = np.random.default_rng(9)
+    X = (0.01 * g.standard_normal((70, 16 if arch == 0 else 9))).astype(np.float32)
+    X[:, 9:] = 0.0
+    X = torch.from_numpy(X).to(gpu)
+    plain = fec.surrogate.material_update(asm, kind[1], X)
+    fec.surrogate.material_update(asm, kind[0], X)
+    assert net.fallbacks() == (0, 70)
+    dout = net.shape[-1]
+    bad = [{o: v} for o in range(dout) for v in (np.nan, np.inf, -np.inf)]
+    bad += [{o: np.inf for o in range(dout)}, {0: np.inf, 3: np.inf, 5: np.inf, 6: -np.inf}]
+    for outputs in bad:
+        v = w.copy()
+        for o, x in outputs.items():
+            v[w.size - dout + o] = x  # the output layer's bias
+        net.set_params(v)
+        Y = fec.surrogate.material_update(asm, kind[0], X)
+        assert net.fallbacks() == (70, 70), outputs
+        assert (Y - plain).abs().max().item() <= 1e-6 * plain.abs().max().item(), outputs
+    # an assembly that accepted every point, then frozen, then the network breaks
+    Uu = torch.from_numpy(0.01 * np.cos(np.arange(asm.dof.unknown_dofs.size))).to(gpu)
+    net.set_params(w)
+    fec.assemble_vector_and_stiffness_(asm, Uu, p)
+    assert net.fallbacks()[0] == 0
+    net.freeze()
+    v = w.copy()
+    v[0] = np.nan
+    net.set_params(v)
+    fec.assemble_vector_and_stiffness_(asm, Uu, p)
+    nfb, npts = net.fallbacks()
+    assert nfb == npts == wl.mesh.num_elements * 8
+    _, ref, pr = _asm(fec, gpu, plain_phys)
+    fec.assemble_vector_and_stiffness_(ref, Uu, pr)
+    for a, b in ((fec.residual(asm), fec.residual(ref)), (asm.stiffness_storage, ref.stiffness_storage)):
+        assert (a - b).abs().max().item() <= 1e-6 * b.abs().max().item()
