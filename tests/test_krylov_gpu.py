@@ -157,3 +157,67 @@ def test_rows_of_loose_nodes(fec, gpu, name):
         assert np.linalg.norm(xg.cpu().numpy() - xs) <= 1e-9 * np.linalg.norm(xs)
         assert abs(res.value - np.linalg.norm(r)) <= 1e-9 * np.linalg.norm(b)
         assert np.array_equal(xg.cpu().numpy()[empty], x[empty])
+
+
+@pytest.mark.parametrize("name", ["quad4 260", "hex8 40 nf1", "quad4 150 nf2", "hex8 25", "hex8 18 roller", "tet10 13"])
+def test_cg_over_many_lines_and_batches(fec, gpu, name):
+    """Matrices of more lines than the product's 1,024 work-groups have lane groups, so that each takes two or three and the last
+    ranges are ragged (quad4 260: 2,129 units of 32 rows; tet10: rows of up to 195 columns, two passes of a lane group), and solves
+    of more iterations than two batches of 8, stopped around their ends or converged. The matrix: -U(0.5, 1.5) off the diagonal,
+    symmetric, diagonal 1.1 times the row's sum, so its condition number is at most 2.1 / 0.1 = 21 after Jacobi scaling and, the
+    row sums within a factor of 13, 273 without. Rounding of k iterations' sums over n <= 7e4 unknowns, taken as random, moves the
+    iterate by condition sqrt(n) k eps: 3e-11 for the 50 iterations that the first condition number allows, 1.2e-9 for the 150 of
+    the second; 2e-9 is asked for."""
+    print(f"[krylov] many lines {name}", flush=True)
+    if name.startswith("tet10"):
+        mesh, nf, fixed = fec.kuhn_tet10_mesh(int(name.split()[1])), 3, {}
+    else:
+        mesh, nf, fixed = _mesh(fec, name)
+    space = fec.FunctionSpace(mesh, "H1Field", "Lagrange")
+    var = fec.ScalarFunction(space, "u") if nf == 1 else fec.VectorFunction(space, "displ")
+    asm = fec.SparseMatrixAssembler(var, sparse_matrix_type="csr", device=0)
+    for d, nodes in fixed.items():
+        mesh.nodeset_nodes[f"_f{d}"] = nodes
+    bcs = [fec.DirichletBC(var.names[d], lambda X, t: 0.0, nset_name=f"_f{d}") for d in fixed]
+    physics = fec.Poisson() if nf == 1 else fec.Mechanics(fec.PlaneStrain() if nf == 2 else None)
+    fec.create_parameters(mesh, asm, physics, dirichlet_bcs=bcs)
+    rp, cv = (t.cpu().numpy() for t in asm.pattern())
+    n = rp.size - 1
+    import scipy.sparse as sp
+    g = np.random.default_rng(4)
+    A = sp.csr_matrix((-0.25 - 0.5 * g.random(cv.size), cv, rp), shape=(n, n))
+    A = (A + A.T).tocsr()
+    A.sort_indices()
+    assert np.array_equal(A.indptr, rp) and np.array_equal(A.indices, cv)
+    rows = np.repeat(np.arange(n), np.diff(rp))
+    A.data[cv == rows] = 0.0
+    A.data[cv == rows] = 1.1 * -np.asarray(A.sum(axis=1)).ravel()
+    vals, diag = torch.from_numpy(A.data).to(gpu), A.diagonal()
+    b, x0 = g.standard_normal(n), g.standard_normal(n)
+    bd = torch.from_numpy(b).to(gpu)
+    tol = 1e-9 * np.linalg.norm(b)
+    P = fec.assembler._ptr
+    for pre in (1, 0):
+        d = 1.0 / diag if pre else np.ones(n)
+        x, r = x0.copy(), b - A @ x0
+        q = d * r
+        rz, k, at = r @ q, 0, {}
+        while np.linalg.norm(r) > tol:
+            at[k] = x.copy(), np.linalg.norm(r)
+            Aq = A @ q
+            a = rz / (q @ Aq)
+            x, r = x + a * q, r - a * Aq
+            new = r @ (d * r)
+            q, rz, k = d * r + new / rz * q, new, k + 1
+        at[k] = x, np.linalg.norm(r)
+        assert 24 < k < 1000
+        for maxit in (0, 7, 8, 9, 16, 17, 24, k - 1, k, k + 1, k + 30):
+            xg = torch.from_numpy(x0).to(gpu)
+            it, res = ctypes.c_int(-1), ctypes.c_double(-1.0)
+            asm.ctx.call("fecx_cg_solve", P(vals), P(bd), P(xg), ctypes.c_double(1e-9), ctypes.c_double(0.0), ctypes.c_int(maxit),
+                         ctypes.c_int(pre), ctypes.byref(it), ctypes.byref(res))
+            want = min(maxit, k)
+            assert it.value == want, (pre, maxit)
+            xs, rs = at[want]
+            assert np.linalg.norm(xg.cpu().numpy() - xs) <= 2e-9 * np.linalg.norm(xs), (pre, maxit)
+            assert abs(res.value - rs) <= 2e-9 * np.linalg.norm(b), (pre, maxit)
