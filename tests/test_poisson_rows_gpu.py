@@ -72,3 +72,28 @@ def test_allocation_free_call_gives_the_same_bits(fec, gpu, counts):
     P = fec.assembler._ptr
     asm.ctx.call("fecx_assemble_vector_matrix_noalloc", P(p.field), P(R), P(K))
     assert torch.equal(R, asm.residual_storage) and torch.equal(K, asm.stiffness_storage)
+
+
+@pytest.mark.parametrize("counts,fixed,source", [((33, 34, 33), "none", "constant"), ((36, 28, 38), "random", "sines"),
+                                                 ((2, 190, 180), "none", "sines"), ((81, 82, 79), "random", "sines")])
+def test_bits_of_the_other_two_phase_kernels(fec, gpu, counts, fixed, source):
+    """The kernels with one lane per element and per row sum in the order of those with 8 lanes each, which an assembly in two
+    pieces and a residual alone still take: the same bits."""
+    print(f"[poisson rows] bits {counts} {fixed} {source}", flush=True)
+    mesh = _brick(fec, *counts)
+    V = fec.FunctionSpace(mesh, "H1Field", "Lagrange")
+    asm = fec.SparseMatrixAssembler(fec.ScalarFunction(V, "u"), sparse_matrix_type="csr", device=gpu.index or 0)
+    bcs = []
+    if fixed == "random":
+        mesh.nodeset_nodes["_bc"] = np.flatnonzero(np.random.default_rng(5).random(mesh.num_nodes) < 0.3) + 1
+        bcs = [fec.DirichletBC("u", lambda X, t: 0.25, nset_name="_bc")]
+    p = fec.create_parameters(mesh, asm, fec.Poisson(source, 1.5), dirichlet_bcs=bcs)
+    Uu = torch.from_numpy(np.cos(0.37 * np.arange(asm.dof.unknown_dofs.size))).to(gpu)
+    fec.assemble_vector_and_stiffness_(asm, Uu, p)
+    R, K = asm.residual_storage.clone(), asm.stiffness_storage.clone()
+    asm.ctx.call("fecx_set_chunks", ctypes.c_int(2))
+    asm.stiffness_storage.fill_(float("nan"))
+    fec.assemble_vector_and_stiffness_(asm, Uu, p)
+    assert torch.equal(asm.residual_storage, R) and torch.equal(asm.stiffness_storage, K)
+    fec.assemble_vector_(asm, fec.residual, Uu, p)
+    assert torch.equal(asm.residual_storage, R)
