@@ -1,17 +1,18 @@
 // MLP building blocks on CDNA4 matrix cores (v_mfma_f32_32x32x16_bf16), shared by the surrogate training kernels
 // and the batched material kernels.
 //
-// Layout ("transposed" formulation): an MFMA tile is 32 samples wide (training: one tile per wavefront; inference: two). A layer computes Z = W H + b with the
-// weights as the MFMA A operand (32 output features x 16 inputs per instruction) and the activations as the B operand
-// (16 inputs x 32 samples). Measured operand layouts on gfx950 (lane l, element i; h = l / 32):
+// Layout ("transposed" formulation): an MFMA tile is 32 samples wide. A layer computes Z = W H + b with the weights as the MFMA
+// A operand (32 output features x 16 inputs per instruction) and the activations as the B operand (16 inputs x 32 samples).
+// Measured operand layouts on gfx950 (lane l, element i; h = l / 32):
 //   A[m = l % 32][k = 8 h + i],  B[k = 8 h + i][n = l % 32],  D register j: [m = 8 (j / 4) + 4 h + j % 4][n = l % 32].
 // A 32-feature output tile in D layout is, after bias + GELU + conversion to BF16, already the B operand of the next
 // layer for two 16-input blocks, provided the next layer's weight columns are stored in the matching order: input block
 // kb = 2 t + s, lane half h, element i holds hidden feature
 //   perm(kb, h, i) = 32 t + 16 s + 8 (i / 4) + 4 h + i % 4.
-// So a whole network runs in registers, with no LDS traffic between layers. The backward pass chains the same way with
-// W^T packed in the same permuted order. The weight-gradient GEMM (sum over samples) uses the same instruction with
-// samples as the reduction dimension.
+// So a wavefront's inference runs in registers, with no LDS traffic between layers (one or two tiles, mlp_hidden). Training
+// gives each wavefront 32 features of a hidden layer and hands these operands round through LDS, backwards too, with W^T packed
+// in the same permuted order (mlp.hip). The weight-gradient GEMM (sum over samples) uses the same instruction with samples as
+// the reduction dimension.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -82,10 +83,6 @@ struct Offs {
   static constexpr int hrows(int l) { return l == 0 ? 32 : A::P[l]; }
 };
 
-// hidden-feature order of a packed B operand (see the header comment)
-__host__ __device__ constexpr int perm_feature(int kb, int h, int i) {
-  return 32 * (kb / 2) + 16 * (kb % 2) + 8 * (i / 4) + 4 * h + i % 4;
-}
 // feature held by D-layout register j of output tile mt in lane half h
 __host__ __device__ constexpr int dreg_feature(int mt, int h, int j) { return 32 * mt + 8 * (j / 4) + 4 * h + j % 4; }
 
@@ -118,56 +115,10 @@ __device__ __forceinline__ float gelu_prime(float z) {
   return fmaf(z * s * (1.0f - s), du, s);
 }
 
-// Z = W_l H + b for one layer; hb holds P[l] / 16 B operands, acc receives P[l+1] / 32 D tiles.
-template <class A, int L>
-__device__ __forceinline__ void mlp_layer(const MlpDev& m, const bf16x8* hb, f32x16* acc, int lane) {
-  constexpr int IN = A::P[L], OUT = A::P[L + 1];
-  const bf16x8* w = m.wf + Offs<A>::wf(L);
-  const float* b = m.bias + Offs<A>::bias(L);
-  const int h = lane >> 5;
-#pragma unroll
-  for (int mt = 0; mt < OUT / 32; ++mt) {
-    f32x16 c;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) c[j] = b[dreg_feature(mt, h, j)];
-#pragma unroll
-    for (int kb = 0; kb < IN / 16; ++kb)
-      c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[(mt * (IN / 16) + kb) * 64 + lane], hb[kb], c, 0, 0, 0);
-    acc[mt] = c;
-  }
-}
-
-// dH = W_l^T dZ for the backward pass (l >= 1); db holds P[l+1] / 16 B operands of dZ_{l+1}.
-template <class A, int L>
-__device__ __forceinline__ void mlp_layer_t(const MlpDev& m, const bf16x8* db, f32x16* acc, int lane) {
-  constexpr int IN = A::P[L + 1], OUT = A::P[L];
-  const bf16x8* w = m.wb + Offs<A>::wb(L);
-#pragma unroll
-  for (int mt = 0; mt < OUT / 32; ++mt) {
-    f32x16 c = {};
-#pragma unroll
-    for (int kb = 0; kb < IN / 16; ++kb)
-      c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[(mt * (IN / 16) + kb) * 64 + lane], db[kb], c, 0, 0, 0);
-    acc[mt] = c;
-  }
-}
-
-// D tiles -> B operands of the next layer (no activation)
-template <int OUT>
-__device__ __forceinline__ void pack_tiles(const f32x16* acc, bf16x8* hb) {
-#pragma unroll
-  for (int mt = 0; mt < OUT / 32; ++mt)
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int i = 0; i < 8; ++i) hb[2 * mt + s][i] = (__bf16)acc[mt][8 * s + i];
-}
-
 // Z = W_l H + b for one hidden layer and T tiles of 32 samples, with the bias, GELU and BF16 packing applied one 32-feature D
 // tile at a time straight into the next layer's B operands: T D tiles (16 registers each) are live instead of P[l+1] / 2
 // registers per tile of samples. Every weight operand is loaded once for the T tiles: the weights of a wavefront come from L2
-// (76 KB for the J2 network, 144 KB for the neo-Hookean one, against 32 KB of L1). Same arithmetic, in the same order, as
-// mlp_layer followed by gelu.
+// (76 KB for the J2 network, 144 KB for the neo-Hookean one, against 32 KB of L1).
 template <class A, int L, int T>
 __device__ __forceinline__ void mlp_layer_gelu(const MlpDev& m, const bf16x8 (&hb)[T][A::P[L] / 16],
                                                bf16x8 (&hn)[T][A::P[L + 1] / 16], int lane) {
@@ -263,17 +214,8 @@ __device__ __forceinline__ void mlp_forward_wave(const MlpDev& m, const float* x
 #pragma unroll
   for (int i = 0; i < 4; ++i) swap_halves(t0.w[i], t1.w[i]);
   const bf16x8 h0[2][1] = {{t0.v}, {t1.v}};
-  bf16x8 h1[2][A::P[1] / 16], h2[2][A::P[2] / 16];
   f32x16 out[2];
-  mlp_layer_gelu<A, 0, 2>(m, h0, h1, lane);
-  mlp_layer_gelu<A, 1, 2>(m, h1, h2, lane);
-  if constexpr (A::NL == 3) {
-    mlp_layer_out<A, 2>(m, h2, out, lane);
-  } else {
-    bf16x8 h3[2][A::P[3] / 16];
-    mlp_layer_gelu<A, 2, 2>(m, h2, h3, lane);
-    mlp_layer_out<A, 2>(m, h3, out, lane);
-  }
+  mlp_hidden<A, 2>(m, h0, out, lane);
 #pragma unroll
   for (int j = 0; j < 8; ++j) {  // features 0-15: lane halves 0 and 1 of the tiles' D registers
     uint32_t a = __float_as_uint(out[0][j]), b = __float_as_uint(out[1][j]);

@@ -595,7 +595,8 @@ __global__ __launch_bounds__(RED_THREADS) __attribute__((amdgpu_waves_per_eu(8, 
 // blocks, 64 for up to 64, and 128 for up to 128 (rows of 65 blocks: 128 lanes with one slot each measured 7.59 ms for
 // the tet10 80^3 reduction against 7.95 ms with 64 lanes in two sweeps, whose second sweep is lane 0 alone; staging all
 // 24 incidences in one pass with 8 loads in flight per lane then took it from 7.82 to 7.21 ms). The scatter kernel
-// has since taken over the 3-field light rows and the tet10 vertex rows of up to 72 blocks; wider rows stay here.
+// has since taken over the light rows of 2 and 3 fields, all light tet10 rows and the tet10 rows of up to 72 blocks; wider tet10
+// rows stay here, on 128 lanes.
 template <int NF, int NNPE>
 static int launch_lpr(const ReduceArgs& a, int maxdeg, hipStream_t s) {
   if (a.p1 <= a.p0) return 0;
@@ -608,7 +609,7 @@ static int launch_lpr(const ReduceArgs& a, int maxdeg, hipStream_t s) {
   int64_t grid = (a.p1 - a.p0 + npw - 1) / npw;
   grid = (grid + 7) / 8 * 8;  // XCD remap needs a multiple of 8
   const unsigned g = (unsigned)grid;
-  if constexpr (NF == 1) {
+  if constexpr (NF == 1 && NNPE != 10) {
     if (lpr == 8) {
       if (sw == 1) reduce_rows_kernel<NF, NNPE, 8, 1><<<g, RED_THREADS, 0, s>>>(a);
       else if (sw == 2) reduce_rows_kernel<NF, NNPE, 8, 2><<<g, RED_THREADS, 0, s>>>(a);
@@ -616,9 +617,19 @@ static int launch_lpr(const ReduceArgs& a, int maxdeg, hipStream_t s) {
       return 0;
     }
   }
-  if (lpr == 32) reduce_rows_kernel<NF, NNPE, 32, 1><<<g, RED_THREADS, 0, s>>>(a);
-  else if (lpr == 64) reduce_rows_kernel<NF, NNPE, 64, 1><<<g, RED_THREADS, 0, s>>>(a);
-  else if (sw == 1) reduce_rows_kernel<NF, NNPE, 128, 1, RED_HEAVY_CH><<<g, RED_THREADS, 0, s>>>(a);
+  if constexpr (NNPE != 10) {  // tet10 rows come here with more than 72 blocks
+    if (lpr == 32) {
+      reduce_rows_kernel<NF, NNPE, 32, 1><<<g, RED_THREADS, 0, s>>>(a);
+      return 0;
+    }
+    if (lpr == 64) {
+      reduce_rows_kernel<NF, NNPE, 64, 1><<<g, RED_THREADS, 0, s>>>(a);
+      return 0;
+    }
+  } else if (lpr != RED_HEAVY_LPR) {
+    return -1;
+  }
+  if (sw == 1) reduce_rows_kernel<NF, NNPE, 128, 1, RED_HEAVY_CH><<<g, RED_THREADS, 0, s>>>(a);
   else reduce_rows_kernel<NF, NNPE, 128, 2, RED_HEAVY_CH><<<g, RED_THREADS, 0, s>>>(a);
   return 0;
 }
