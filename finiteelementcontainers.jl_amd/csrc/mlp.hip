@@ -384,8 +384,10 @@ __device__ void repack_param(const MlpPack& pk, int64_t p, float w) {
 }
 
 // The last work-group sums the n loss partials by one wavefront in a fixed order (lane l takes partials l, l + 64, ..., then a
-// fixed xor tree across lanes), so every run gives the same bits. The chunks of a parameter are added in ascending order with
-// eight loads on their way (64 chunks of the neo-Hookean network: 14 us one load at a time, now 5).
+// fixed xor tree across lanes), so every run gives the same bits. The chunks of a parameter are added in a fixed order too, by
+// eights whose loads are on their way together (64 chunks of the neo-Hookean network: 14 us one load at a time, now 5) and
+// whose sum is a tree: 64 rounded additions one after the other are 1.2e-7 off the exact sum, these 4.9e-8 (4,096 samples,
+// relative 2-norm; 16 chunks of 256 samples one after the other were 6.8e-8 off).
 template <int ARCH>
 __global__ void mlp_update_kernel(UpdateArgs a) {
   if (a.loss && blockIdx.x == gridDim.x - 1) {
@@ -406,8 +408,7 @@ __global__ void mlp_update_kernel(UpdateArgs a) {
       float v[8];
 #pragma unroll
       for (int k = 0; k < 8; ++k) v[k] = a.part[(int64_t)(c + k) * a.np + p];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) g += v[k];
+      g += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
     }
     for (; c < a.nchunk; ++c) g += a.part[(int64_t)c * a.np + p];
     if (a.grad) a.grad[p] = g;

@@ -34,3 +34,28 @@ def test_gradient_at_the_edges(fec, mlpref, gpu, arch, n):
     assert err <= 2e-2, err
     loss2, grad2 = net.gradient(X, T)  # the same bits again
     assert loss2 == loss and torch.equal(grad2, grad)
+
+
+@pytest.mark.parametrize("arch", [0, 1])
+@pytest.mark.parametrize("n", [1024, 4096])
+def test_sums_over_chunks(fec, gpu, arch, n):
+    """The gradient of n samples, whose chunks have 64 samples each, against the FP64 mean of the gradients of those 64: their
+    products are the same (n and 64 are powers of two, so the scaling of dz is exact). m additions one after the other of random
+    terms are off by 0.41 sqrt(m / 2) roundings of 2^-24; the sum by eights has 8 of them at most and trees of three levels, 0.41
+    sqrt(3): 1.1 together, and 1.5 roundings, 9e-8 of the gradient's 2-norm, are asked for (64 additions: 2.3)."""
+    print(f"[network gradient] sums of {n} samples, arch {arch}", flush=True)
+    physics = fec.J2Surrogate(200.0, 0.3, 0.25, 2.0) if arch == 0 else fec.NeoHookeanSurrogate(1.0, 0.5)
+    wl = fec.workloads.j2_hex8(2)
+    var = fec.VectorFunction(fec.FunctionSpace(wl.mesh, "H1Field", "Lagrange"), "displ")
+    asm = fec.SparseMatrixAssembler(var, sparse_matrix_type="csr", device=gpu.index or 0)
+    fec.create_parameters(wl.mesh, asm, physics)
+    net = fec.Surrogate(asm, arch, seed=3)
+    g = np.random.default_rng(6)
+    X = torch.from_numpy(g.standard_normal((n, 16 if arch == 0 else 9)).astype(np.float32)).to(gpu)
+    T = torch.from_numpy(g.standard_normal((n, net.shape[-1])).astype(np.float32)).to(gpu)
+    whole = net.gradient(X, T)[1].double()
+    pieces = torch.zeros_like(whole)
+    for k in range(0, n, 64):
+        pieces += net.gradient(X[k:k + 64], T[k:k + 64])[1].double()
+    pieces /= n // 64
+    assert (whole - pieces).norm().item() <= 1.5 * 2.0 ** -24 * pieces.norm().item()
