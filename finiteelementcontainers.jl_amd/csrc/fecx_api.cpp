@@ -947,12 +947,12 @@ int fecx_assemble_mass_action(fecx_ctx* ctx, double density, const double* V, do
 
 int fecx_update_fields(fecx_ctx* ctx, const double* bc, const double* Uu, double* U, const double* Vu, double* V) {
   return guard(ctx, [&] {
+    check_device(ctx);
     require(ctx->has_dofs, FECX_ERR_STATE, "fecx_set_dofs has not been called");
     const bool unknowns = !ctx->unknown_dofs.empty(), fixed = bc && !ctx->dirichlet.empty();
     require(Uu || !unknowns, FECX_ERR_ARG, "Uu is NULL");
     require(U || !(unknowns || fixed), FECX_ERR_ARG, "U is NULL");
     require(Vu || !V || !unknowns, FECX_ERR_ARG, "V without Vu");
-    check_device(ctx);
     const fecx::DofMap m = dof_map(ctx);
     fecx::launch_update_fields(m, ctx->dirichlet.empty() ? nullptr : bc, Uu, U, Vu, V, ctx->stream);
     HIPCHK(hipGetLastError());
@@ -965,9 +965,9 @@ int fecx_update_field_unknowns(fecx_ctx* ctx, const double* Uu, double* U) {
 
 int fecx_update_field_dirichlet(fecx_ctx* ctx, const double* vals, double* U) {
   return guard(ctx, [&] {
+    check_device(ctx);
     require(ctx->has_dofs, FECX_ERR_STATE, "fecx_set_dofs has not been called");
     require((vals && U) || ctx->dirichlet.empty(), FECX_ERR_ARG, "vals or U is NULL");
-    check_device(ctx);
     fecx::launch_scatter_indexed((int64_t)ctx->dirichlet.size(), get<int64_t>(ctx, "dirichlet_idx"), vals, U,
                                  ctx->stream);
     HIPCHK(hipGetLastError());
@@ -976,9 +976,9 @@ int fecx_update_field_dirichlet(fecx_ctx* ctx, const double* vals, double* U) {
 
 int fecx_extract_field_unknowns(fecx_ctx* ctx, const double* U, double* Uu) {
   return guard(ctx, [&] {
+    check_device(ctx);
     require(ctx->has_dofs, FECX_ERR_STATE, "fecx_set_dofs has not been called");
     require((U && Uu) || ctx->unknown_dofs.empty(), FECX_ERR_ARG, "U or Uu is NULL");
-    check_device(ctx);
     fecx::launch_extract_unknowns(dof_map(ctx), U, Uu, ctx->stream);
     HIPCHK(hipGetLastError());
   });

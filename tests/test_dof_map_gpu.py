@@ -51,3 +51,33 @@ def test_update_and_extract(fec, gpu, nx, ny, nf, share, condensed):
     out = torch.full((len(free),), float("nan"), dtype=torch.float64, device=gpu)
     c.call("fecx_extract_field_unknowns", P(d["U"]), P(out))
     assert np.array_equal(out.cpu().numpy(), host["U"][free])
+
+
+@pytest.mark.parametrize("fixed", ["none", "some", "all"])
+def test_null_arrays_are_refused(fec, gpu, fixed):
+    """A field call refuses NULL (code -1) in the place of an array that it would read or write; arrays that the dofs leave
+    untouched may be NULL."""
+    mesh = fec.StructuredMesh("hex", (0, 0, 0), (1, 1, 1), (2, 2, 2))
+    dirichlet = np.arange(1, {"none": 1, "some": 4, "all": 9}[fixed], dtype=np.int64)
+    c = fec._lib.Context(0)
+    fec.assembler._set_mesh(c, mesh, fec._lib.HEX8)
+    c.call("fecx_set_dofs", ctypes.c_int(1), fec.assembler._host_ptr(dirichlet) if len(dirichlet) else None,
+           ctypes.c_int64(len(dirichlet)))
+    arrays = torch.zeros((5, 8), dtype=torch.float64, device=gpu)
+    x = [fec.assembler._ptr(t) for t in arrays.unbind()]
+    free, bc = fixed != "all", fixed != "none"
+    calls = [("fecx_update_fields", (x[0], x[1], x[2], x[3], x[4]), False), ("fecx_update_fields", (None, x[1], x[2], None, None), False),
+             ("fecx_update_fields", (None, x[1], x[2], x[3], None), False), ("fecx_update_fields", (x[0], None, x[2], x[3], x[4]), free),
+             ("fecx_update_fields", (x[0], x[1], None, x[3], x[4]), True), ("fecx_update_fields", (None, x[1], None, x[3], x[4]), free),
+             ("fecx_update_fields", (x[0], x[1], x[2], None, x[4]), free), ("fecx_update_field_unknowns", (x[0], x[1]), False),
+             ("fecx_update_field_unknowns", (None, x[1]), free), ("fecx_update_field_unknowns", (x[0], None), free),
+             ("fecx_update_field_dirichlet", (None, x[1]), bc), ("fecx_update_field_dirichlet", (x[0], None), bc),
+             ("fecx_extract_field_unknowns", (None, x[1]), free), ("fecx_extract_field_unknowns", (x[0], None), free)]
+    for name, args, refused in calls:
+        if not refused:
+            c.call(name, *args)
+            continue
+        with pytest.raises(fec.FECXError) as ei:
+            c.call(name, *args)
+        assert ei.value.code == -1, name
+    torch.cuda.synchronize()

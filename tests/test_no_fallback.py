@@ -33,27 +33,3 @@ def test_host_context_refuses_kernels(fec):
         hp.ctx.call("fecx_assemble_vector", U.ctypes.data_as(__import__("ctypes").c_void_p),
                     R.ctypes.data_as(__import__("ctypes").c_void_p))
     assert "host-only" in str(ei.value)
-
-
-@pytest.mark.parametrize("fixed", ["none", "some", "all"])
-def test_field_calls_refuse_null_arrays(fec, fixed):
-    """A field call that would read or write an array refuses NULL in its place (code -1) before anything runs; arrays that the
-    dofs leave untouched may be NULL, and such calls get as far as the host-only context's own refusal (code -2)."""
-    import ctypes
-    mesh = fec.StructuredMesh("hex", (0, 0, 0), (1, 1, 1), (2, 2, 2))
-    dirichlet = np.arange(1, {"none": 1, "some": 4, "all": 9}[fixed])
-    ctx = fec.HostPattern(mesh, 1, dirichlet.astype(np.int64)).ctx
-    a = np.zeros(8)
-    x = a.ctypes.data_as(ctypes.c_void_p)
-    free, bc = fixed != "all", fixed != "none"
-    calls = [("fecx_update_fields", (x, x, x, x, x), False), ("fecx_update_fields", (None, x, x, None, None), False),
-             ("fecx_update_fields", (None, x, x, x, None), False), ("fecx_update_fields", (x, None, x, x, x), free),
-             ("fecx_update_fields", (x, x, None, x, x), True), ("fecx_update_fields", (None, x, None, x, x), free),
-             ("fecx_update_fields", (x, x, x, None, x), free), ("fecx_update_field_unknowns", (x, x), False),
-             ("fecx_update_field_unknowns", (None, x), free), ("fecx_update_field_unknowns", (x, None), free),
-             ("fecx_update_field_dirichlet", (None, x), bc), ("fecx_update_field_dirichlet", (x, None), bc),
-             ("fecx_extract_field_unknowns", (None, x), free), ("fecx_extract_field_unknowns", (x, None), free)]
-    for name, args, refused in calls:
-        with pytest.raises(fec.FECXError) as ei:
-            ctx.call(name, *args)
-        assert ei.value.code == (-1 if refused else -2), (name, args)
