@@ -1191,8 +1191,8 @@ void fused_hex8_kernel(ElementArgs args, FusedArgs f) {
 // (not deterministic), colouring in colour order.
 // PART: the values go to the dof-level CSR of a partial Dirichlet set (csr_row). A look at the map per entry, whether there is
 // one or not, keeps the coloured design from loading a block's entries together: steps of neo-Hookean 96^3 17.1 ms against 9.3, on
-// rollers 17.2 against 9.9, 6^3 277 us against 204, on rollers 355 against 270 (every position of a mapped row loaded first, or one
-// block ahead: 295).
+// rollers 17.2 against 7.9, 6^3 277 us against 204, on rollers 355 against 254 (mapped rows with every position loaded first, or one
+// block ahead, and the other rows entry by entry: 295; both kinds of rows by one list of positions: 267, but 13.4 ms at 96^3).
 template <int NF, int PHYS, int ATOMIC, bool PART>
 __global__ __launch_bounds__(ELEM_THREADS) __attribute__((amdgpu_waves_per_eu(2, 8)))
 void scatter_hex8_kernel(ElementArgs args, FusedArgs f, int colour) {
@@ -1250,35 +1250,43 @@ void scatter_hex8_kernel(ElementArgs args, FusedArgs f, int colour) {
       const int slot = __popc(mask & ((1u << d) - 1u));
       const PairRef pr = pair_ref(8, a, b);
       const float* blk = work.K + grp * KW + pr.slot * NB;
-      auto word = [&](int i, int k) { return (double)blk[pr.ab ? i * NF + k : k * NF + i]; };
-      if constexpr (PART) {
-        if (row.map) {  // all positions, then all values (the entries are distinct), then the stores
-          int at[NB];
-          double x[NB];
+      auto word = [&](int c) { return (double)blk[pr.ab ? c : c % NF * NF + c / NF]; };
+      double* dst = row.vals + NF * slot;
+      if constexpr (!PART) {
 #pragma unroll
-          for (int c = 0; c < NB; ++c) at[c] = row.map[((c / NF) * deg + slot) * NF + c % NF];
-          if constexpr (!ATOMIC) {
+        for (int c = 0; c < NB; ++c) {
+          double* p = dst + (int64_t)(c / NF) * NF * deg + c % NF;
+          if (ATOMIC) atomicAdd(p, word(c));
+          else *p += word(c);
+        }
+        continue;
+      }
+      // the entries of a block are distinct: all positions, then all values, then the stores
+      int at[NB];
+      double x[NB];
+      if (row.map) {
 #pragma unroll
-            for (int c = 0; c < NB; ++c) x[c] = at[c] >= 0 ? row.vals[at[c]] : 0.0;
-          }
+        for (int c = 0; c < NB; ++c) at[c] = row.map[((c / NF) * deg + slot) * NF + c % NF];
 #pragma unroll
-          for (int c = 0; c < NB; ++c)
-            if (at[c] >= 0) {
-              if constexpr (ATOMIC) atomicAdd(row.vals + at[c], word(c / NF, c % NF));
-              else row.vals[at[c]] = x[c] + word(c / NF, c % NF);
-            }
-          continue;
+        for (int c = 0; c < NB; ++c)
+          if (!ATOMIC) x[c] = at[c] >= 0 ? row.vals[at[c]] : 0.0;
+#pragma unroll
+        for (int c = 0; c < NB; ++c) {
+          if (at[c] < 0) continue;
+          if (ATOMIC) atomicAdd(row.vals + at[c], word(c));
+          else row.vals[at[c]] = x[c] + word(c);
+        }
+      } else {
+#pragma unroll
+        for (int c = 0; c < NB; ++c)
+          if (!ATOMIC) x[c] = dst[(c / NF) * NF * deg + c % NF];
+#pragma unroll
+        for (int c = 0; c < NB; ++c) {
+          double* p = dst + (c / NF) * NF * deg + c % NF;
+          if (ATOMIC) atomicAdd(p, word(c));
+          else *p = x[c] + word(c);
         }
       }
-      double* dst = row.vals + NF * slot;
-#pragma unroll
-      for (int i = 0; i < NF; ++i)
-#pragma unroll
-        for (int k = 0; k < NF; ++k) {
-          double* p = dst + (int64_t)i * NF * deg + k;
-          if (ATOMIC) atomicAdd(p, word(i, k));
-          else *p += word(i, k);
-        }
     }
   }
   if (bad) raise_flag(args.flag);
