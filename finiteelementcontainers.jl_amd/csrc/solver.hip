@@ -91,17 +91,21 @@ __device__ __forceinline__ void sum_partials2(const double* p, const double* q, 
 
 // ------------------------------------------------------------------ products with the matrix
 // A "line" is what one lane group multiplies: the NF rows of a free node (NF columns per block share one column index and
-// one gather of the vector across the NF rows), or (NF = 0) one row of a dof-level CSR. L lanes per line, lane l taking
+// one gather of the vector across the NF rows), or (DOF_ROWS) one row of a dof-level CSR. L lanes per line, lane l taking
 // columns l, l + L, ..., U of them in flight together: L U covers the rows of a structured mesh (hex8: 27 columns of one
 // field, 81 of three; quad4: 18 of two), so such a line costs one chain of loads (pointer, column, vector), and the next
 // line's pointer and columns are fetched under the current one's (cg_product_kernel). Wider rows (tet10: up to 195) loop.
 // Lanes for 81 columns, whole solve of an elastic hex8 40 x 32 x 36 block (1,187 iterations): 16 lanes x 6 columns 37.0 ms
 // (spills at 4 waves per SIMD), 32 x 3 31.4 ms; for 27 columns (Poisson hex8 36^3, 155 iterations): 8 lanes x 4 2.13 ms,
-// 16 x 2 2.36 ms, 32 x 1 2.62 ms.
+// 16 x 2 2.36 ms, 32 x 1 2.62 ms; for the 18 of a dof-level row of two fields (300 x 401 nodes on rollers, 100 iterations): 8 lanes
+// x 3 2.64 ms, 32 x 3 6.50 (SpMV 26.9 against 48.6 us).
+constexpr int DOF_ROWS = 0, DOF_ROWS_2 = -2;  // a row of a dof-level CSR, of 3 fields and of 2
 template <int NF>
 struct LineShape {
-  static constexpr int L = NF == 1 ? 8 : (NF == 2 ? 16 : 32), U = NF == 1 ? 4 : (NF == 2 ? 2 : 3);
-  static constexpr int R = NF == 0 ? 1 : NF, B = R;  // rows and columns per block
+  static constexpr bool DOF = NF <= 0;
+  static constexpr int L = NF == 1 || NF == DOF_ROWS_2 ? 8 : (NF == 2 ? 16 : 32);
+  static constexpr int U = NF == 1 ? 4 : (NF == 2 ? 2 : 3);
+  static constexpr int R = DOF ? 1 : NF, B = R;  // rows and columns per block
   static constexpr int GPW = SV_THREADS / L;         // lines per work-group
 };
 template <int NF>
@@ -113,7 +117,7 @@ template <int NF>
 __device__ __forceinline__ LinePtr<NF> line_ptr(const CsrView& A, uint32_t g, uint32_t lines) {
   LinePtr<NF> p{0, 0};
   if (g < lines) {
-    const int64_t* q = (NF == 0 ? A.rptr : A.bptr) + g;
+    const int64_t* q = (LineShape<NF>::DOF ? A.rptr : A.bptr) + g;
     const int64_t rb = q[0];
     p.n = (int)(q[1] - rb) * LineShape<NF>::B;
     p.rb = p.n > 0 ? rb : 0;  // the last rows, empty, start where the matrix ends
@@ -127,7 +131,7 @@ __device__ __forceinline__ int line_col(const LinePtr<NF>& p, int j) { return j 
 template <int NF>
 __device__ __forceinline__ void line_index(const CsrView& A, const LinePtr<NF>& p, int j0, uint32_t (&idx)[LineShape<NF>::U]) {
   using S = LineShape<NF>;
-  const int32_t* col = (NF == 0 ? A.rcol : A.bcol) + p.rb;
+  const int32_t* col = (S::DOF ? A.rcol : A.bcol) + p.rb;
 #pragma unroll
   for (int u = 0; u < S::U; ++u) {
     const int j = line_col<NF>(p, j0 + u * S::L);
@@ -437,8 +441,9 @@ __global__ void axpy_kernel(int64_t n, double a, const double* x, double* y) {
 static int vec_groups(int64_t n) { return (int)std::min<int64_t>((n + SV_THREADS - 1) / SV_THREADS, CG_PARTS); }
 
 template <class F>
-static void by_line(int nf, const CsrView& A, F f) {  // f(integral constant NF): 0 for a dof-level CSR
-  if (A.rptr) f(std::integral_constant<int, 0>());
+static void by_line(int nf, const CsrView& A, F f) {  // f(integral constant NF)
+  if (A.rptr && nf == 2) f(std::integral_constant<int, DOF_ROWS_2>());
+  else if (A.rptr) f(std::integral_constant<int, DOF_ROWS>());
   else if (nf == 1) f(std::integral_constant<int, 1>());
   else if (nf == 2) f(std::integral_constant<int, 2>());
   else f(std::integral_constant<int, 3>());

@@ -89,10 +89,23 @@ def test_spmv_and_cg_iterations(fec, gpu, name):
         assert abs(res.value - np.linalg.norm(r)) <= 1e-9 * np.linalg.norm(b)
 
 
+def _quads(fec, name):
+    """(mesh, 2, fixed) of a square or of quadrilaterals around a point (rows of up to 2 (2 m + 1) columns), on rollers"""
+    m = int(name.split()[1])
+    if name.startswith("quadfan"):
+        t = np.pi * np.arange(2 * m) / m
+        ring = np.stack([np.cos(t), np.sin(t)], axis=1) * np.where(np.arange(2 * m) % 2, 1.4, 1.0)[:, None]
+        conn = np.array([[0, 1 + 2 * i, 2 + 2 * i, 1 + (2 * i + 2) % (2 * m)] for i in range(m)]) + 1
+        mesh = fec.BlockMesh(np.concatenate([np.zeros((1, 2)), ring]), [("b", conn)], "QUAD4")
+    else:
+        mesh = fec.StructuredMesh("quad", (0.0, 0.0), (1.0, 1.0), (m + 1, m + 1))
+    return mesh, 2, {d: np.flatnonzero(mesh.coords[:, d] < mesh.coords[:, d].min() + 1e-12) + 1 for d in range(2)}
+
+
 def _loose(fec, name):
     """(mesh, nf, fixed): a brick or square with a loose node (of no element) before, between and after the others', the last
     rows of the matrix being empty; "alone": every node of an element is fixed, so that the matrix has no entry"""
-    m, nf, fixed = _mesh(fec, name.replace(" alone", ""))
+    m, nf, fixed = _quads(fec, name) if name.startswith("quad") and "roller" in name else _mesh(fec, name.replace(" alone", ""))
     n = m.num_nodes
     at = np.concatenate([[-1], np.arange(n // 2), [-1], np.arange(n // 2, n), [-1, -1]])  # new node -> old node
     new = np.empty(n, np.int64)
@@ -105,7 +118,9 @@ def _loose(fec, name):
     return mesh, nf, fixed, np.flatnonzero(at < 0)
 
 
-@pytest.mark.parametrize("name", ["hex8 3 nf1", "hex8 3", "hex8 3 roller", "quad4 5 nf2", "hex8 2 nf1 alone", "hex8 2 alone"])
+@pytest.mark.parametrize("name", ["hex8 3 nf1", "hex8 3", "hex8 3 roller", "quad4 5 nf2", "quad4 2 nf2 roller", "quad4 7 nf2 roller",
+                                  "quadfan 5 nf2 roller", "quadfan 6 nf2 roller", "quadfan 40 nf2 roller", "hex8 2 nf1 alone",
+                                  "hex8 2 alone"])
 def test_rows_of_loose_nodes(fec, gpu, name):
     """Nodes that no element touches have empty rows: a product of zero, a unit preconditioner, and an unknown that CG leaves at its
     start (b is zero there, or the matrix has no entry). Tolerances as above."""
@@ -159,7 +174,8 @@ def test_rows_of_loose_nodes(fec, gpu, name):
         assert np.array_equal(xg.cpu().numpy()[empty], x[empty])
 
 
-@pytest.mark.parametrize("name", ["quad4 260", "hex8 40 nf1", "quad4 150 nf2", "hex8 25", "hex8 18 roller", "tet10 13"])
+@pytest.mark.parametrize("name", ["quad4 260", "hex8 40 nf1", "quad4 150 nf2", "quad4 130 nf2 roller", "hex8 25", "hex8 18 roller",
+                                  "tet10 13"])
 def test_cg_over_many_lines_and_batches(fec, gpu, name):
     """Matrices of more lines than the product's 1,024 work-groups have lane groups, so that each takes two or three and the last
     ranges are ragged (quad4 260: 2,129 units of 32 rows; tet10: rows of up to 195 columns, two passes of a lane group), and solves
@@ -172,7 +188,7 @@ def test_cg_over_many_lines_and_batches(fec, gpu, name):
     if name.startswith("tet10"):
         mesh, nf, fixed = fec.kuhn_tet10_mesh(int(name.split()[1])), 3, {}
     else:
-        mesh, nf, fixed = _mesh(fec, name)
+        mesh, nf, fixed = _quads(fec, name) if name.startswith("quad") and "roller" in name else _mesh(fec, name)
     space = fec.FunctionSpace(mesh, "H1Field", "Lagrange")
     var = fec.ScalarFunction(space, "u") if nf == 1 else fec.VectorFunction(space, "displ")
     asm = fec.SparseMatrixAssembler(var, sparse_matrix_type="csr", device=0)
